@@ -11,6 +11,8 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PACKAGE_ROOT = Path(__file__).resolve().parent
@@ -23,7 +25,8 @@ LIB_PATH = LIB_DIR / "libseqattn_hip.so"
 PROBE_LIB_PATH = LIB_DIR / "libseqattn_probe.so"
 ARCH = "gfx950"
 
-SOURCES = ("sa_kernels.hip", "sa_pipeline.cpp")
+SOURCES = ("sa_kernels.hip", "sa_update_d32.hip", "sa_update_d64.hip", "sa_update_d128.hip", "sa_update_d256.hip",
+           "sa_pipeline.cpp")
 PROBE_SOURCES = ("sa_probe.hip",)
 
 # Device-side flags.  Packed FP32 VALU instructions are disabled for all
@@ -60,19 +63,7 @@ def build(verbose: bool = False) -> Path:
     return LIB_PATH
 
 
-def _link(sources, target: Path, verbose: bool) -> None:
-    LIB_DIR.mkdir(parents=True, exist_ok=True)
-    tmp = target.with_suffix(".so.tmp")
-    cmd = [
-        hipcc(),
-        *HIP_FLAGS,
-        f"-I{INCLUDE}",
-        f"-I{CSRC}",
-        "-shared",
-        *(str(CSRC / name) for name in sources),
-        "-o",
-        str(tmp),
-    ]
+def _run(cmd, verbose: bool) -> None:
     if verbose:
         print(" ".join(cmd), flush=True)
     result = subprocess.run(cmd, capture_output=True, text=True)
@@ -85,6 +76,22 @@ def _link(sources, target: Path, verbose: bool) -> None:
         raise RuntimeError(f"hipcc failed ({result.returncode}):\n{stderr}")
     if verbose and stderr.strip():
         print(stderr, file=sys.stderr)
+
+
+def _link(sources, target: Path, verbose: bool) -> None:
+    """Compile the sources in parallel and link them into ``target``."""
+    LIB_DIR.mkdir(parents=True, exist_ok=True)
+    tmp = target.with_suffix(".so.tmp")
+    with tempfile.TemporaryDirectory() as work:
+        objects = [Path(work) / f"{Path(name).stem}.o" for name in sources]
+        with ThreadPoolExecutor(max_workers=4) as pool:
+            for done in [
+                pool.submit(_run, [hipcc(), *HIP_FLAGS, f"-I{INCLUDE}", f"-I{CSRC}", "-c", str(CSRC / name), "-o",
+                                   str(obj)], verbose)
+                for name, obj in zip(sources, objects)
+            ]:
+                done.result()
+        _run([hipcc(), f"--offload-arch={ARCH}", "-shared", *map(str, objects), "-o", str(tmp)], verbose)
     os.replace(tmp, target)
 
 

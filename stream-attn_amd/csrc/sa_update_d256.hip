@@ -1,0 +1,14 @@
+// The update kernel's variants for head_dim padded to 256.  INT8 K/V covers
+// head_dim <= 128: with head_dim 256 the 16-bit stages and the raw staging
+// would not fit in LDS together.
+#include "sa_update_kernel.h"
+
+namespace sa {
+
+hipError_t launch_update_d256(const UpdateParams& p, int mode, int rows, int dtype, hipStream_t stream) {
+  (void)mode;
+  return rows == 128 ? launch_variant<256, 1, kRows>(p, dtype, stream)
+                     : launch_variant<256, 2, kRows>(p, dtype, stream);
+}
+
+}  // namespace sa
