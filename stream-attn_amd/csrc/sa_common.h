@@ -66,6 +66,9 @@ struct FusedOutput {
   float* lse;
   int64_t lse_sh, lse_off;
 };
+// Flag of launch_update (beside SA_FLAG_*): another update launch of about
+// this size runs beside this one on the other stream.
+constexpr int32_t kLaunchOverlapped = 1 << 16;
 int32_t launch_update(const void* q, const void* k, const void* v, float* m, float* l, float* acc,
                       int64_t sq_t, int64_t sq_h, int64_t sk_t, int64_t sk_h, int64_t sv_t,
                       int64_t sv_h, int64_t ss_t, int64_t ss_h, int64_t sa_t, int64_t sa_h,
@@ -97,7 +100,7 @@ int32_t launch_finalize(const float* acc, const float* m, const float* l, void* 
 // tiled_state: m, l and acc are the pipeline's own buffers in the row-group
 // layout (16-row groups, lane order; see the update kernels), not strided.
 
-// Queries per workgroup of the update kernel for this head_dim: launches that
-// split a Q block split it at a multiple of this.
+// Row granularity at which launches split a Q block: the update kernel's
+// widest workgroup for this head_dim, or a fraction of it.
 int32_t update_block_rows(int32_t head_dim);
 }  // namespace sa

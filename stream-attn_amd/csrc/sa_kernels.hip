@@ -9,6 +9,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <mutex>
@@ -129,11 +130,66 @@ __global__ __launch_bounds__(256) void transpose_v_kernel(const TransposeParams 
   }
 }
 
-hipError_t launch_update_variant(const UpdateParams& p, int mode, int dtype, hipStream_t stream) {
+constexpr int kCUs = 256;
+
+// Modelled time (in the units of kVariants) of `heads` x the query blocks of
+// v.rows queries, from the measured time per tile.  Blocks of equal length
+// run in rounds of one (or two) workgroups per CU; under a causal mask long
+// blocks start first and short ones fill in behind them, and a launch that
+// shares the chip with another one fills in behind that.  No launch ends
+// before its longest block.  Over 60 drawn shapes the choice was within 3% of
+// the best variant's time on average.
+double variant_time(const UpdateVariant& v, int64_t q_tokens, int64_t kv_tokens, int64_t heads, bool causal,
+                    int64_t first_visible, bool overlapped) {
+  const int64_t blocks = (q_tokens + v.rows - 1) / v.rows;
+  const int64_t n = blocks * heads;
+  const auto tiles = [&](int64_t keys) {
+    return (double)((std::max<int64_t>(0, std::min(keys, kv_tokens)) + kTileKeys - 1) / kTileKeys);
+  };
+  // Keys seen by the last and the first block.
+  const double longest = causal ? tiles(first_visible + q_tokens - 1) : tiles(kv_tokens);
+  const double shortest = causal ? tiles(first_visible + std::min<int64_t>(v.rows, q_tokens) - 1) : longest;
+  if (n <= kCUs) return longest * v.one;
+  if (causal || overlapped) {
+    // Longest first: within one shortest block of an even spread, and no
+    // worse than rounds of falling length.
+    const double slot = v.two ? v.two : v.one;
+    const double slots = v.two ? 2 * kCUs : kCUs;
+    const double even = 0.5 * (longest + shortest) * n / slots * slot;
+    const double rounds = std::ceil(n / slots);
+    const double in_rounds = rounds * slot * (longest - (longest - shortest) * 0.5 * (rounds - 1) * slots / n);
+    return std::max(longest * v.one, overlapped ? even : std::min(in_rounds, even + shortest * slot));
+  }
+  if (!v.two) return (double)((n + kCUs - 1) / kCUs) * longest * v.one;
+  const int64_t full = n / (2 * kCUs), rest = n % (2 * kCUs);
+  const double last = rest == 0 ? 0.0 : rest <= kCUs ? v.one : v.one + (v.two - v.one) * (rest - kCUs) / (double)kCUs;
+  return (full * v.two + last) * longest;
+}
+
+// Queries per workgroup.  A query's bits do not depend on it, so it is chosen
+// for time alone: wide workgroups read each K/V tile for more queries (bf16,
+// head_dim 128: 6.7 ns per query and tile at 384 queries, 7.8 at 128), narrow
+// ones fill the chip with few queries and waste less of a last round or of a
+// causal diagonal.  1,009 queries over 61,312 keys x 32 heads: 384 queries
+// are 96 workgroups, 128 are 256.
+int choose_rows(const UpdateParams& p, int d, int mode, bool overlapped) {
+  int rows = kVariants[d][0].rows;
+  double best = 0.0;
+  for (UpdateVariant v : kVariants[d]) {
+    if (!v.rows) continue;
+    // The INT8 staging of head_dim 128 leaves LDS for one workgroup.
+    if (mode == kInt8 && d == 2) v.two = 0;
+    const double t = variant_time(v, p.q_tokens, p.kv_tokens, p.q_heads, p.causal,
+                                  (int64_t)p.q_local_offset + p.causal_shift - p.kv_local_offset + 1, overlapped);
+    // Ties go to the wider workgroup (less traffic).
+    if (best == 0.0 || t <= best) best = t, rows = v.rows;
+  }
+  return rows;
+}
+
+hipError_t launch_update_variant(const UpdateParams& p, int mode, int dtype, bool overlapped, hipStream_t stream) {
   const int d = p.head_dim <= 32 ? 0 : p.head_dim <= 64 ? 1 : p.head_dim <= 128 ? 2 : 3;
-  // The widest workgroup, unless half of one fills every CU once at most.
-  int rows = d == 2 ? 384 : 256;
-  if (d == 3 && ((int64_t)p.q_tokens + 127) / 128 * p.q_heads <= 256) rows = 128;
+  const int rows = choose_rows(p, d, mode, overlapped);
   switch (d) {
     case 0: return launch_update_d32(p, mode, rows, dtype, stream);
     case 1: return launch_update_d64(p, mode, rows, dtype, stream);
@@ -249,7 +305,8 @@ int32_t launch_update(const void* q, const void* k, const void* v, float* m, flo
     set_error("transposed V needs head_dim 128, an initializing launch and a padded [heads][128][keys] layout");
     return SA_ERR_INVALID_ARGUMENT;
   }
-  const hipError_t err = launch_update_variant(p, v_transposed ? kTransposedV : kRows, dtype, stream);
+  const hipError_t err = launch_update_variant(p, v_transposed ? kTransposedV : kRows, dtype,
+                                               (flags & kLaunchOverlapped) != 0, stream);
   return err == hipSuccess ? 0 : hip_status(err, "update kernel launch");
 }
 
@@ -333,7 +390,7 @@ int32_t launch_update_int8(const void* q, const void* k, const void* v, const vo
   p.tiled_state = tiled_state ? 1 : 0;
   p.causal = (flags & SA_FLAG_CAUSAL) != 0;
   p.init = (flags & SA_FLAG_INITIALIZE) != 0;
-  const hipError_t err = launch_update_variant(p, kInt8, dtype, stream);
+  const hipError_t err = launch_update_variant(p, kInt8, dtype, false, stream);
   return err == hipSuccess ? 0 : hip_status(err, "int8 update kernel launch");
 }
 
@@ -572,8 +629,8 @@ int32_t sa_update_attention_state(const void* q, const void* k, const void* v, f
   return sa::launch_update(q, k, v, running_max, running_sum, accumulator, stride_qt, stride_qh,
                            stride_kt, stride_kh, stride_vt, stride_vh, stride_st, stride_sh,
                            stride_at, stride_ah, q_tokens, kv_tokens, q_heads, kv_heads, head_dim,
-                           q_local_offset, kv_local_offset, causal_shift, softmax_scale, flags,
-                           dtype, static_cast<hipStream_t>(stream));
+                           q_local_offset, kv_local_offset, causal_shift, softmax_scale,
+                           flags & (SA_FLAG_CAUSAL | SA_FLAG_INITIALIZE), dtype, static_cast<hipStream_t>(stream));
 }
 
 int32_t sa_update_attention_state_int8(

@@ -413,7 +413,8 @@ int32_t apply_span(sa_pipeline* p, const void* q, int64_t sq_t, int64_t sq_h, co
     const int64_t position = (int64_t)kv_local_offset + start;
     if (!*initialize && position >= visible_end) break;
     const int32_t n = std::min(p->kv_chunk, kv_tokens - start);
-    const int32_t flags = (causal ? SA_FLAG_CAUSAL : 0) | (*initialize ? SA_FLAG_INITIALIZE : 0);
+    const int32_t flags = (causal ? SA_FLAG_CAUSAL : 0) | (*initialize ? SA_FLAG_INITIALIZE : 0) |
+                          (two ? sa::kLaunchOverlapped : 0);
     const bool fuse = fused_last != nullptr && start == last_start;
     if (fuse && fused_done) *fused_done = true;
     int32_t rc;
@@ -971,7 +972,7 @@ int32_t fused_merge_keys(const sa_pipeline* p, int64_t k_length) {
 int32_t launch_unit(sa_pipeline* p, const void* q, int64_t sq_t, const void* k, int64_t sk_t, const void* v,
                     int64_t sv_t, int64_t sv_h, int32_t q_tokens, int32_t kv_tokens, int32_t q_heads,
                     int32_t kv_heads, int32_t causal_shift, double scale, int32_t causal, int32_t merge_keys,
-                    const sa::FusedOutput& fused, bool v_transposed, hipStream_t stream) {
+                    const sa::FusedOutput& fused, bool v_transposed, bool overlapped, hipStream_t stream) {
   TraceRange range(p->trace, "seqattn:fused_update");
   if (p->timing) {
     if (p->t_used == p->t_start.size()) {
@@ -983,7 +984,8 @@ int32_t launch_unit(sa_pipeline* p, const void* q, int64_t sq_t, const void* k, 
     }
     SA_HIP_RETURN(hipEventRecord(p->t_start[p->t_used], stream));
   }
-  const int32_t flags = (causal ? SA_FLAG_CAUSAL : 0) | SA_FLAG_INITIALIZE;
+  const int32_t flags =
+      (causal ? SA_FLAG_CAUSAL : 0) | SA_FLAG_INITIALIZE | (overlapped ? sa::kLaunchOverlapped : 0);
   const int32_t rc = sa::launch_update(q, k, v, nullptr, nullptr, nullptr, sq_t, p->head_dim, sk_t, p->head_dim,
                                        sv_t, sv_h, 0, 0, 0, 0, q_tokens, kv_tokens, q_heads, kv_heads, p->head_dim,
                                        0, 0, causal_shift, scale, flags, p->dtype, stream, merge_keys, &fused,
@@ -1191,7 +1193,7 @@ int32_t run_head_groups(sa_pipeline* p, const char* qh, const char* kh, const ch
                                      (int64_t)gk * p->head_dim, vt ? static_cast<const char*>(p->set_vt[b]) : vseg,
                                      vt ? t_pad : (int64_t)gk * p->head_dim, vt ? 128 * t_pad : p->head_dim,
                                      (int32_t)q_length, (int32_t)k_length, gq, gk, (int32_t)(k_length - q_length),
-                                     scale, causal, fused_merge_keys(p, k_length), fused, vt, cs);
+                                     scale, causal, fused_merge_keys(p, k_length), fused, vt, join.active, cs);
       if (rc != 0) return rc;
       chunks += (k_length + p->kv_chunk - 1) / p->kv_chunk;
     }
