@@ -413,10 +413,10 @@ int32_t sa_pipeline_stream_kv_gather_int8(sa_pipeline* pipeline, const void* con
  * each block is finalized straight into out (and lse when non-NULL, layout
  * [q_heads, total_q] with row stride lse_stride_h).  When kv_chunk_tokens is
  * a multiple of 64 and out is 16-byte aligned with strides that are multiples
- * of 8, each segment is one update launch over all of its queries and keys
- * that finalizes in its epilogue and merges the row sums at every chunk
- * boundary, so the result equals sa_pipeline_run's bit for bit; the state
- * buffers are then untouched.  Enqueued on compute_stream; returns without
+ * of 8, one update launch covers all queries and keys of a segment (or of up
+ * to 32 segments together), finalizes in its epilogue and merges the row sums
+ * at every chunk boundary, so the result equals sa_pipeline_run's bit for bit;
+ * the state buffers are then untouched.  Enqueued on compute_stream; returns without
  * waiting.  The reference accepts host
  * tensors only (validation.py:13-14); this is the device-input extension.
  */
@@ -432,10 +432,11 @@ int32_t sa_pipeline_run_resident(sa_pipeline* pipeline, const void* q, const voi
 /*
  * Attach caller-owned device scratch for sa_pipeline_run_resident (NULL and 0
  * detach it).  No counterpart in the reference.  With head_dim 128, a fused
- * resident launch whose segment has kv_tokens keys first copies V into it,
- * transposed per K/V head ([kv_heads][128][keys padded to a multiple of 64],
- * 16-bit), when kv_heads * 128 * roundup(kv_tokens, 64) * 2 bytes fit; the
- * update kernel then reads V^T fragments with half the LDS instructions.
+ * resident launch whose segment has kv_tokens keys and at least 65,536
+ * queries x query heads per K/V head first copies V into it, transposed per
+ * K/V head (128 x the keys padded to a multiple of 64, 16-bit), when
+ * kv_heads * 128 * roundup(kv_tokens, 64) * 2 bytes fit; the update kernel
+ * then reads V^T fragments with half the LDS instructions.
  * Results are identical with or without it.  The pipeline keeps the pointer
  * until it is replaced or the pipeline is destroyed; runs on one pipeline
  * share it, in stream order.
@@ -516,8 +517,9 @@ int32_t sa_pipeline_kernel_busy(sa_pipeline* pipeline, double* busy_ms, double* 
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  It computes what sa_pipeline_run_resident computes for
  * head_dim 128 with transposed-V scratch attached, bit for bit (same
- * launches: a V transpose per segment, then one fused update launch whose
- * row sums merge at every kv_chunk_tokens boundary), but the transposed V
+ * launches: fused update launches whose row sums merge at every
+ * kv_chunk_tokens boundary, V transposed before those of large segments), but
+ * the transposed V
  * lives in a fixed 64 MiB device array inside the library (one per GPU,
  * held until the process ends) instead of caller-provided scratch.
  * Limits: head_dim 128; per segment kv_heads * 128 * (keys rounded up to

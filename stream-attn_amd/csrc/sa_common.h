@@ -6,8 +6,10 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdarg>
+#include <cstdint>
 #include <cstdio>
 #include <string>
+#include <vector>
 
 #include "seqattn_hip.h"
 
@@ -54,6 +56,33 @@ class DeviceGuard {
     if (sa_err_ != hipSuccess) return sa::hip_status(sa_err_, #call); \
   } while (0)
 
+// Segments launched together, relative to the first one's rows.
+namespace sa {
+struct Segment {
+  int32_t q0, k0, q_len, k_len;
+};
+struct SegmentGroup {
+  std::vector<Segment> segments;
+  int64_t q0 = 0, k0 = 0;  // the packed rows that q0 = k0 = 0 stands for
+  // False (and not added) where the group's rows would not fit 32 bits.
+  bool add(int64_t q_start, int64_t q_length, int64_t k_start, int64_t k_length) {
+    if (segments.empty()) q0 = q_start, k0 = k_start;
+    if (q_start - q0 + q_length > INT32_MAX || k_start - k0 + k_length > INT32_MAX) return false;
+    segments.push_back({(int32_t)(q_start - q0), (int32_t)(k_start - k0), (int32_t)q_length, (int32_t)k_length});
+    return true;
+  }
+  int64_t q_span() const { return (int64_t)segments.back().q0 + segments.back().q_len; }
+  int64_t k_span() const { return (int64_t)segments.back().k0 + segments.back().k_len; }
+};
+// Whether a segment is worth a transposed copy of V before its launch (where
+// there is scratch for one).  The copy moves V twice, one launch of its own;
+// its fragments then take half the LDS instructions.  Measured with head_dim
+// 128: 0.3-0.7% faster at 65,536 and more queries x query heads per K/V head,
+// no gain at 32,768, 2-8% slower at 8,192 and below, where it also cannot
+// join a launch with other segments.
+inline bool transposes_v(int64_t q_length, int64_t group) { return q_length * group >= 65536; }
+}  // namespace sa
+
 // Kernel entry points shared between the kernel and pipeline translation units.
 namespace sa {
 // Output of an update launch that also finalizes its rows (launch_update with
@@ -65,6 +94,12 @@ struct FusedOutput {
   int64_t so_t, so_h;
   float* lse;
   int64_t lse_sh, lse_off;
+  // With num_segments > 0 the launch covers these segments, each with its own
+  // queries (rows [q0, q0 + q_len) of q, out and lse) and keys (rows [k0,
+  // k0 + k_len) of k and v, bottom-right causal); q_tokens and kv_tokens are
+  // then the rows that q and k span.  V in place only, no state loaded.
+  const Segment* segments = nullptr;
+  int32_t num_segments = 0;
 };
 // Flag of launch_update (beside SA_FLAG_*): another update launch of about
 // this size runs beside this one on the other stream.

@@ -13,6 +13,7 @@
 #include <cmath>
 #include <cstdint>
 #include <mutex>
+#include <vector>
 
 #include "sa_common.h"
 #include "sa_update_kernel.h"
@@ -132,38 +133,50 @@ __global__ __launch_bounds__(256) void transpose_v_kernel(const TransposeParams 
 
 constexpr int kCUs = 256;
 
-// Modelled time (in the units of kVariants) of `heads` x the query blocks of
+int64_t tiles_of(int64_t keys) { return (std::max<int64_t>(0, keys) + kTileKeys - 1) / kTileKeys; }
+
+// Modelled time (in the units of kVariants) of the launch with workgroups of
 // v.rows queries, from the measured time per tile.  Blocks of equal length
-// run in rounds of one (or two) workgroups per CU; under a causal mask long
-// blocks start first and short ones fill in behind them, and a launch that
-// shares the chip with another one fills in behind that.  No launch ends
-// before its longest block.  Over 60 drawn shapes the choice was within 3% of
-// the best variant's time on average.
-double variant_time(const UpdateVariant& v, int64_t q_tokens, int64_t kv_tokens, int64_t heads, bool causal,
-                    int64_t first_visible, bool overlapped) {
-  const int64_t blocks = (q_tokens + v.rows - 1) / v.rows;
-  const int64_t n = blocks * heads;
-  const auto tiles = [&](int64_t keys) {
-    return (double)((std::max<int64_t>(0, std::min(keys, kv_tokens)) + kTileKeys - 1) / kTileKeys);
+// run in rounds of one (or two) workgroups per CU; under a causal mask and
+// with several segments long blocks start first and short ones fill in behind
+// them, and a launch that shares the chip with another one fills in behind
+// that.  No launch ends before its longest block.  Over 60 drawn shapes the
+// choice was within 3% of the best variant's time on average.
+double variant_time(const UpdateVariant& v, const UpdateParams& p, bool overlapped) {
+  double longest = 0, shortest = 0, work = 0, n = 0;
+  const auto add = [&](int64_t q_len, int64_t k_len, int64_t first_visible) {
+    const double blocks = (double)((q_len + v.rows - 1) / v.rows) * p.q_heads;
+    // Tiles of the last and the first block.
+    const double last = tiles_of(p.causal ? std::min(k_len, first_visible + q_len - 1) : k_len);
+    const double first =
+        p.causal ? tiles_of(std::min(k_len, first_visible + std::min<int64_t>(v.rows, q_len) - 1)) : last;
+    longest = std::max(longest, last);
+    shortest = n == 0 ? first : std::min(shortest, first);
+    work += 0.5 * (first + last) * blocks;
+    n += blocks;
   };
-  // Keys seen by the last and the first block.
-  const double longest = causal ? tiles(first_visible + q_tokens - 1) : tiles(kv_tokens);
-  const double shortest = causal ? tiles(first_visible + std::min<int64_t>(v.rows, q_tokens) - 1) : longest;
-  if (n <= kCUs) return longest * v.one;
-  if (causal || overlapped) {
-    // Longest first: within one shortest block of an even spread, and no
-    // worse than rounds of falling length.
-    const double slot = v.two ? v.two : v.one;
-    const double slots = v.two ? 2 * kCUs : kCUs;
-    const double even = 0.5 * (longest + shortest) * n / slots * slot;
-    const double rounds = std::ceil(n / slots);
-    const double in_rounds = rounds * slot * (longest - (longest - shortest) * 0.5 * (rounds - 1) * slots / n);
-    return std::max(longest * v.one, overlapped ? even : std::min(in_rounds, even + shortest * slot));
+  if (p.segments > 1) {
+    for (int s = 0; s < p.segments; ++s)
+      add(p.segment[s].q_len, p.segment[s].k_len, p.segment[s].k_len - p.segment[s].q_len + 1);
+  } else {
+    add(p.q_tokens, p.kv_tokens, (int64_t)p.q_local_offset + p.causal_shift - p.kv_local_offset + 1);
   }
-  if (!v.two) return (double)((n + kCUs - 1) / kCUs) * longest * v.one;
-  const int64_t full = n / (2 * kCUs), rest = n % (2 * kCUs);
-  const double last = rest == 0 ? 0.0 : rest <= kCUs ? v.one : v.one + (v.two - v.one) * (rest - kCUs) / (double)kCUs;
-  return (full * v.two + last) * longest;
+  if (n <= kCUs) return longest * v.one;
+  const double slots = v.two ? 2 * kCUs : kCUs, slot = v.two ? v.two : v.one;
+  const double even = work / slots * slot;
+  if (overlapped) return std::max(longest * v.one, even);
+  if (longest == shortest) {
+    const double full = std::floor(n / slots), rest = n - full * slots;
+    const double partly = rest == 0     ? 0.0
+                          : rest <= kCUs ? v.one
+                                         : v.one + (slot - v.one) * (rest - kCUs) / kCUs;
+    return (full * slot + partly) * longest;
+  }
+  // Longest first: within one shortest block of an even spread, and no worse
+  // than rounds of falling length.
+  const double rounds = std::ceil(n / slots);
+  const double in_rounds = rounds * slot * (longest - (longest - shortest) * 0.5 * (rounds - 1) * slots / n);
+  return std::max(longest * v.one, std::min(in_rounds, even + shortest * slot));
 }
 
 // Queries per workgroup.  A query's bits do not depend on it, so it is chosen
@@ -174,15 +187,14 @@ double variant_time(const UpdateVariant& v, int64_t q_tokens, int64_t kv_tokens,
 // are 96 workgroups, 128 are 256.
 int choose_rows(const UpdateParams& p, int d, int mode, bool overlapped) {
   int rows = kVariants[d][0].rows;
-  double best = 0.0;
+  double best = -1.0;
   for (UpdateVariant v : kVariants[d]) {
     if (!v.rows) continue;
     // The INT8 staging of head_dim 128 leaves LDS for one workgroup.
     if (mode == kInt8 && d == 2) v.two = 0;
-    const double t = variant_time(v, p.q_tokens, p.kv_tokens, p.q_heads, p.causal,
-                                  (int64_t)p.q_local_offset + p.causal_shift - p.kv_local_offset + 1, overlapped);
+    const double t = variant_time(v, p, overlapped);
     // Ties go to the wider workgroup (less traffic).
-    if (best == 0.0 || t <= best) best = t, rows = v.rows;
+    if (best < 0.0 || t <= best) best = t, rows = v.rows;
   }
   return rows;
 }
@@ -196,6 +208,45 @@ hipError_t launch_update_variant(const UpdateParams& p, int mode, int dtype, boo
     case 2: return launch_update_d128(p, mode, rows, dtype, stream);
     default: return launch_update_d256(p, mode, rows, dtype, stream);
   }
+}
+
+// The segments of one call in launches of up to kMaxSegments, those with the
+// most keys first: the workgroups of one launch run side by side, where a
+// launch per segment left CUs idle at the end of each (11 ragged segments of
+// 1,800 tokens x 32 heads on average: 11 launches of 38-86 us one after the
+// other).
+int32_t launch_segments(UpdateParams p, const FusedOutput& fused, int dtype, bool overlapped, hipStream_t stream) {
+  std::vector<Segment> order;
+  order.reserve(fused.num_segments);
+  for (int32_t s = 0; s < fused.num_segments; ++s)
+    if (fused.segments[s].q_len > 0) order.push_back(fused.segments[s]);
+  std::stable_sort(order.begin(), order.end(), [](const Segment& a, const Segment& b) { return a.k_len > b.k_len; });
+  const int64_t most = (int64_t)INT32_MAX / 8;  // workgroups of a launch
+  for (size_t at = 0; at < order.size();) {
+    int64_t workgroups = 0;
+    p.segments = 0;
+    while (at < order.size() && p.segments < kMaxSegments) {
+      const int64_t more = ((int64_t)order[at].q_len + 127) / 128 * p.q_heads;
+      if (p.segments > 0 && workgroups + more > most) break;
+      workgroups += more;
+      p.segment[p.segments++] = order[at++];
+    }
+    UpdateParams one = p;
+    if (p.segments == 1) {
+      const Segment& seg = p.segment[0];
+      one.q += (int64_t)seg.q0 * p.sq_t;
+      one.k += (int64_t)seg.k0 * p.sk_t;
+      one.v += (int64_t)seg.k0 * p.sv_t;
+      one.out += (int64_t)seg.q0 * p.so_t;
+      one.lse_off += seg.q0;
+      one.q_tokens = seg.q_len;
+      one.kv_tokens = seg.k_len;
+      one.causal_shift = seg.k_len - seg.q_len;
+    }
+    const hipError_t err = launch_update_variant(one, kRows, dtype, overlapped, stream);
+    if (err != hipSuccess) return hip_status(err, "update kernel launch");
+  }
+  return 0;
 }
 
 inline bool aligned(const void* ptr, uintptr_t n) { return (reinterpret_cast<uintptr_t>(ptr) % n) == 0; }
@@ -292,7 +343,10 @@ int32_t launch_update(const void* q, const void* k, const void* v, float* m, flo
     p.lse_off = fused->lse_off;
   }
   // Workgroup numbering is 32-bit: at least 128 queries per workgroup.
-  if (((int64_t)q_tokens + 127) / 128 * q_heads > (int64_t)INT32_MAX / 8) {
+  int64_t longest_q = fused != nullptr && fused->num_segments > 0 ? 0 : q_tokens;
+  for (int32_t s = 0; fused != nullptr && s < fused->num_segments; ++s)
+    longest_q = std::max<int64_t>(longest_q, fused->segments[s].q_len);
+  if ((longest_q + 127) / 128 * q_heads > (int64_t)INT32_MAX / 8) {
     set_error("sa_update_attention_state: q_tokens * q_heads too large for one launch");
     return SA_ERR_INVALID_ARGUMENT;
   }
@@ -305,8 +359,15 @@ int32_t launch_update(const void* q, const void* k, const void* v, float* m, flo
     set_error("transposed V needs head_dim 128, an initializing launch and a padded [heads][128][keys] layout");
     return SA_ERR_INVALID_ARGUMENT;
   }
-  const hipError_t err = launch_update_variant(p, v_transposed ? kTransposedV : kRows, dtype,
-                                               (flags & kLaunchOverlapped) != 0, stream);
+  const bool overlapped = (flags & kLaunchOverlapped) != 0;
+  if (fused != nullptr && fused->num_segments > 0) {
+    if (v_transposed || !starts_state) {
+      set_error("a launch over segments reads V in place and loads no state");
+      return SA_ERR_INVALID_ARGUMENT;
+    }
+    return launch_segments(p, *fused, dtype, overlapped, stream);
+  }
+  const hipError_t err = launch_update_variant(p, v_transposed ? kTransposedV : kRows, dtype, overlapped, stream);
   return err == hipSuccess ? 0 : hip_status(err, "update kernel launch");
 }
 
@@ -590,30 +651,41 @@ int32_t sa_run_resident_noalloc(const void* q, const void* k, const void* v, voi
   const char* kd = static_cast<const char*>(k);
   const char* vd = static_cast<const char*>(v);
   char* od = static_cast<char*>(out);
+  // The launch sequence of sa_pipeline_run_resident's fused path with the
+  // scratch in place of the attached one: per segment of enough queries V
+  // transposed (zero keys up to the 64-key tile), then one update launch over
+  // it that finalizes in its epilogue with the row sums merged at every K/V
+  // chunk boundary; the other segments together.  All launches are on
+  // `stream`, so a later segment's transpose starts after this segment's
+  // update has read the scratch.
+  const auto launch = [&](const char* v_seg, int64_t sv_t, int64_t sv_h, int64_t q_start, int64_t q_length,
+                          int64_t k_start, int64_t k_length, const sa::FusedOutput& fused, bool transposed) {
+    return sa::launch_update(qd + q_start * stride_qt * 2, kd + k_start * stride_kt * 2, v_seg, nullptr, nullptr,
+                             nullptr, stride_qt, stride_qh, stride_kt, stride_kh, sv_t, sv_h, 0, 0, 0, 0,
+                             (int32_t)q_length, (int32_t)k_length, q_heads, kv_heads, 128, 0, 0,
+                             (int32_t)(k_length - q_length), softmax_scale,
+                             (causal ? SA_FLAG_CAUSAL : 0) | SA_FLAG_INITIALIZE, dtype, hs, kv_chunk_tokens, &fused,
+                             transposed);
+  };
+  sa::SegmentGroup together;
   for (int32_t s = 0; s < num_segments; ++s) {
     const int64_t q_start = cu_seqlens_q[s], k_start = cu_seqlens_k[s];
     const int64_t q_length = cu_seqlens_q[s + 1] - q_start, k_length = cu_seqlens_k[s + 1] - k_start;
     if (q_length == 0) continue;
-    // The launch sequence of sa_pipeline_run_resident's fused path with the
-    // scratch in place of the attached one: V transposed (zero keys up to
-    // the 64-key tile), then one update launch over the segment that
-    // finalizes in its epilogue with the row sums merged at every K/V chunk
-    // boundary.  Both launches are on `stream`, so a later segment's
-    // transpose starts after this segment's update has read the scratch.
+    if (!sa::transposes_v(q_length, q_heads / kv_heads) && together.add(q_start, q_length, k_start, k_length)) continue;
     const int64_t t_pad = (k_length + 63) / 64 * 64;
-    const char* v_seg = vd + k_start * stride_vt * 2;
-    rc = sa::launch_transpose_v(v_seg, stride_vt, stride_vh, (int32_t)k_length, kv_heads, 128, vt, t_pad, hs);
+    rc = sa::launch_transpose_v(vd + k_start * stride_vt * 2, stride_vt, stride_vh, (int32_t)k_length, kv_heads, 128,
+                                vt, t_pad, hs);
     if (rc != 0) return rc;
     const sa::FusedOutput fused{od + q_start * stride_ot * 2, stride_ot, stride_oh, lse, lse_stride_h, q_start};
-    rc = sa::launch_update(qd + q_start * stride_qt * 2, kd + k_start * stride_kt * 2, vt, nullptr, nullptr,
-                           nullptr, stride_qt, stride_qh, stride_kt, stride_kh, t_pad, 128 * t_pad, 0, 0, 0, 0,
-                           (int32_t)q_length, (int32_t)k_length, q_heads, kv_heads, 128, 0, 0,
-                           (int32_t)(k_length - q_length), softmax_scale,
-                           (causal ? SA_FLAG_CAUSAL : 0) | SA_FLAG_INITIALIZE, dtype, hs, kv_chunk_tokens, &fused,
-                           true);
+    rc = launch(static_cast<const char*>(vt), t_pad, 128 * t_pad, q_start, q_length, k_start, k_length, fused, true);
     if (rc != 0) return rc;
   }
-  return 0;
+  if (together.segments.empty()) return 0;
+  const sa::FusedOutput fused{od + together.q0 * stride_ot * 2, stride_ot, stride_oh, lse, lse_stride_h, together.q0,
+                              together.segments.data(), (int32_t)together.segments.size()};
+  return launch(vd + together.k0 * stride_vt * 2, stride_vt, stride_vh, together.q0, together.q_span(), together.k0,
+                together.k_span(), fused, false);
 }
 
 int32_t sa_update_attention_state(const void* q, const void* k, const void* v, float* running_max,

@@ -1742,6 +1742,8 @@ int32_t sa_pipeline_run_resident(sa_pipeline* p, const void* q, const void* k, c
   const char* vd = static_cast<const char*>(v);
   char* od = static_cast<char*>(out);
   const int64_t qt_stride = (int64_t)p->q_heads * p->head_dim;
+  sa::SegmentGroup together;
+  int32_t together_merge = 0;  // the same for every segment that is launched fused
   for (int32_t s = 0; s < num_segments; ++s) {
     const int64_t q_start = cu_seqlens_q[s], q_stop = cu_seqlens_q[s + 1];
     const int64_t k_start = cu_seqlens_k[s], k_stop = cu_seqlens_k[s + 1];
@@ -1774,26 +1776,32 @@ int32_t sa_pipeline_run_resident(sa_pipeline* p, const void* q, const void* k, c
       // sa_pipeline_run's bit for bit, with no state round trips, no
       // per-launch tails and no finalize launches.  Stats count the Q blocks
       // and chunks of the chunked schedule.
-      const sa::FusedOutput fused{seg_out, stride_ot, stride_oh, lse, lse_stride_h, q_start};
-      // With head_dim 128 and enough attached scratch, V is first copied
-      // transposed (keys padded to whole tiles), which the update kernel
-      // reads with half the LDS instructions for the same operands.
+      // With head_dim 128, enough attached scratch and enough queries
+      // (transposes_v), V is first copied transposed (keys padded to whole
+      // tiles), which the update kernel reads with half the LDS instructions
+      // for the same operands; the other segments go together in one launch
+      // after the loop.
       const int64_t t_pad = (k_length + 63) / 64 * 64;
       const int64_t vt_bytes = (int64_t)p->kv_heads * 128 * t_pad * 2;
       const bool vt = p->head_dim == 128 && p->vt_scratch != nullptr && vt_bytes <= p->vt_scratch_bytes &&
-                      t_pad < (1 << 24);
-      int32_t rc = 0;
-      if (vt) {
-        rc = sa::launch_transpose_v(src.v, src.sv_t, src.sv_h, (int32_t)k_length, p->kv_heads, p->head_dim,
-                                    p->vt_scratch, t_pad, compute);
+                      t_pad < (1 << 24) && sa::transposes_v(q_length, p->q_heads / p->kv_heads);
+      if (vt || !together.add(q_start, q_length, k_start, k_length)) {
+        int32_t rc = 0;
+        if (vt) {
+          rc = sa::launch_transpose_v(src.v, src.sv_t, src.sv_h, (int32_t)k_length, p->kv_heads, p->head_dim,
+                                      p->vt_scratch, t_pad, compute);
+          if (rc != 0) return rc;
+        }
+        const sa::FusedOutput fused{seg_out, stride_ot, stride_oh, lse, lse_stride_h, q_start};
+        rc = launch_timed(p, qd + q_start * stride_qt * 2, stride_qt, stride_qh, src.k, src.sk_t, src.sk_h,
+                          vt ? static_cast<const char*>(p->vt_scratch) : src.v, vt ? t_pad : src.sv_t,
+                          vt ? 128 * t_pad : src.sv_h, (int32_t)q_length, (int32_t)k_length, 0, 0, causal_shift,
+                          softmax_scale, (causal ? SA_FLAG_CAUSAL : 0) | SA_FLAG_INITIALIZE, compute, merge,
+                          &fused, 0, vt);
         if (rc != 0) return rc;
+      } else {
+        together_merge = merge;
       }
-      rc = launch_timed(p, qd + q_start * stride_qt * 2, stride_qt, stride_qh, src.k, src.sk_t, src.sk_h,
-                        vt ? static_cast<const char*>(p->vt_scratch) : src.v, vt ? t_pad : src.sv_t,
-                        vt ? 128 * t_pad : src.sv_h, (int32_t)q_length, (int32_t)k_length, 0, 0, causal_shift,
-                        softmax_scale, (causal ? SA_FLAG_CAUSAL : 0) | SA_FLAG_INITIALIZE, compute, merge,
-                        &fused, 0, vt);
-      if (rc != 0) return rc;
       const int64_t block = p->head_groups ? q_length
                                            : pass_rows(q_length, p->q_chunk, sa::update_block_rows(p->head_dim));
       for (int64_t qs = q_start; qs < q_stop; qs += block) {
@@ -1826,6 +1834,16 @@ int32_t sa_pipeline_run_resident(sa_pipeline* p, const void* q, const void* k, c
       if (rc != 0) return rc;
       add_stats(stats, 0, 0, 1, 0, n);
     }
+  }
+  if (!together.segments.empty()) {
+    const sa::FusedOutput fused{od + together.q0 * stride_ot * 2, stride_ot, stride_oh, lse, lse_stride_h,
+                                together.q0, together.segments.data(), (int32_t)together.segments.size()};
+    const int32_t rc = launch_timed(p, qd + together.q0 * stride_qt * 2, stride_qt, stride_qh,
+                                    kd + together.k0 * stride_kt * 2, stride_kt, stride_kh,
+                                    vd + together.k0 * stride_vt * 2, stride_vt, stride_vh, (int32_t)together.q_span(),
+                                    (int32_t)together.k_span(), 0, 0, 0, softmax_scale,
+                                    (causal ? SA_FLAG_CAUSAL : 0) | SA_FLAG_INITIALIZE, compute, together_merge, &fused);
+    if (rc != 0) return rc;
   }
   return 0;
 }

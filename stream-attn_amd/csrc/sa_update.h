@@ -59,6 +59,7 @@
 
 #include <cstdint>
 
+#include "sa_common.h"
 #include "seqattn_hip.h"
 
 namespace sa {
@@ -66,6 +67,24 @@ namespace sa {
 // How K and V arrive: 16-bit rows, 16-bit K rows with V transposed per K/V
 // head, INT8 rows with scales.
 enum KVMode { kRows = 0, kTransposedV = 1, kInt8 = 2 };
+
+// How workgroups are numbered (hardware block b runs on XCD b % 8).
+enum Numbering {
+  // Each XCD takes an eighth of the heads of every segment, so the
+  // workgroups resident on one XCD share few heads' K/V in its L2.
+  kHeadsPerXcd = 0,
+  // Each XCD takes a contiguous eighth of the workgroups: one segment without
+  // a mask whose heads are no multiple of 8.
+  kRunsPerXcd = 1,
+  // Consecutive workgroups go to consecutive XCDs: workgroups of unequal
+  // length (a causal mask, segments) whose heads are no multiple of 8, of
+  // which a contiguous run would give some XCD more than its share of long
+  // ones (measured: 1.7x the runs' rate on one causal head, 1.14x on 12).
+  kDealt = 2,
+};
+
+// Segments of one launch: the table travels in the kernel's arguments.
+constexpr int kMaxSegments = 32;
 
 struct UpdateParams {
   const uint16_t* q;
@@ -78,9 +97,9 @@ struct UpdateParams {
   int32_t q_tokens, kv_tokens, group, head_dim, q_heads;
   int32_t q_local_offset, kv_local_offset, causal_shift;
   int32_t causal, init;
-  int32_t q_blocks;       // workgroups per query head
-  int32_t xcd_run;        // ceil(q_blocks * q_heads / 8)
-  int32_t deal_blocks;    // causal, q_heads not a multiple of 8: every XCD takes every eighth block
+  int32_t numbering;      // Numbering
+  int32_t slots;          // workgroups of the launch (of one XCD, for kHeadsPerXcd)
+  int32_t xcd_run;        // kRunsPerXcd: ceil(slots / 8)
   float scale_log2;
   // INT8 K/V only: fp16 scales, element (group, kv_head) at
   // scales[group * s?s_g + kv_head * s?s_h], group = (scale_offset + key) >> scale_shift.
@@ -109,6 +128,12 @@ struct UpdateParams {
   // State in the pipeline's row-group layout (state_block) instead of the
   // strided [token][head] layout given by ss_* / sa_*.
   int32_t tiled_state;
+  // With segments > 1 the launch covers that many, instead of q_tokens
+  // queries over kv_tokens keys: their rows as in sa::Segment, and the first
+  // workgroup number (see slots) of each.
+  int32_t segments;
+  int32_t first[kMaxSegments];
+  Segment segment[kMaxSegments];
 };
 
 constexpr int kTileKeys = 64;
@@ -123,10 +148,10 @@ struct UpdateVariant {
 constexpr int kHeadDims = 4;  // 32, 64, 128, 256
 constexpr int kMaxVariants = 3;
 constexpr UpdateVariant kVariants[kHeadDims][kMaxVariants] = {
-    {{128, 605, 920}, {256, 930, 1549}, {0, 0, 0}},
-    {{128, 765, 1220}, {256, 1180, 2030}, {0, 0, 0}},
-    {{128, 1180, 2000}, {256, 1835, 0}, {384, 2590, 0}},
-    {{128, 2310, 0}, {256, 3400, 0}, {0, 0, 0}},
+    {{128, 605, 920}, {256, 930, 1550}, {0, 0, 0}},
+    {{128, 800, 1245}, {256, 1245, 2070}, {0, 0, 0}},
+    {{128, 1250, 2040}, {256, 1905, 0}, {384, 2620, 0}},
+    {{128, 2460, 0}, {256, 3505, 0}, {0, 0, 0}},
 };
 
 // One launch with the head-dim's variant of `rows` queries per workgroup.

@@ -150,21 +150,35 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
   __shared__ __attribute__((aligned(1024))) uint8_t lds_qa[kStagingBytes];
   __shared__ __attribute__((aligned(1024))) uint8_t lds_qb[kStagingBytes];
 
-  // XCD-aware numbering: hardware block b runs on XCD b % 8; consecutive
-  // logical workgroups (same head, neighbouring query blocks) share an XCD.
-  // Under a causal mask later query blocks see more keys: they are dealt
-  // first so that the short blocks fill the end of the launch.  Unless the
-  // launch's heads are a multiple of 8 (then each XCD's run holds whole
-  // heads and the runs are kept), a contiguous run would give some XCD more
-  // than its share of long blocks, so in causal launches every XCD takes
-  // every eighth block instead (measured: 1.7x the runs' rate on one head,
-  // 1.14x on 12).
+  const SA_CONSTANT UpdateParams* args = (const SA_CONSTANT UpdateParams*)__builtin_amdgcn_kernarg_segment_ptr();
+
+  // Workgroup -> (segment, head, query block), numbered segment by segment
+  // and head by head (see Numbering).  Under a causal mask later query blocks
+  // see more keys: they come first so that the short blocks fill the end of
+  // the launch.
   const int b = blockIdx.x;
-  const int logical = p.deal_blocks ? b : (b & 7) * p.xcd_run + (b >> 3);
-  if (logical >= p.q_blocks * p.q_heads) return;
-  const int head = logical / p.q_blocks;
-  const int in_head = logical - head * p.q_blocks;
-  const int q_block = (p.causal ? p.q_blocks - 1 - in_head : in_head) * BLOCK_M;
+  int slot = p.numbering == kDealt ? b : b >> 3;
+  if (p.numbering == kRunsPerXcd) slot += (b & 7) * p.xcd_run;
+  if (slot >= p.slots) return;
+  int q_tokens = p.q_tokens, kv_tokens = p.kv_tokens, causal_shift = p.causal_shift;
+  int q0 = 0, k0 = 0;
+  if (p.segments > 1) {
+    // Every lane looks at one segment's first number.
+    const int at = threadIdx.x & 63;
+    const bool before = at < p.segments && args->first[at & (kMaxSegments - 1)] <= slot;
+    const int s = __builtin_amdgcn_readfirstlane(__popcll(__ballot(before)) - 1);
+    slot -= __builtin_amdgcn_readfirstlane(args->first[s]);
+    q0 = __builtin_amdgcn_readfirstlane(args->segment[s].q0);
+    k0 = __builtin_amdgcn_readfirstlane(args->segment[s].k0);
+    q_tokens = __builtin_amdgcn_readfirstlane(args->segment[s].q_len);
+    kv_tokens = __builtin_amdgcn_readfirstlane(args->segment[s].k_len);
+    causal_shift = kv_tokens - q_tokens;
+  }
+  const int q_blocks = (q_tokens + BLOCK_M - 1) / BLOCK_M;
+  const int head_slot = slot / q_blocks;
+  const int head = head_slot + (p.numbering == kHeadsPerXcd ? (b & 7) * (p.q_heads >> 3) : 0);
+  const int in_head = slot - head_slot * q_blocks;
+  const int q_block = (p.causal ? q_blocks - 1 - in_head : in_head) * BLOCK_M;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -174,18 +188,18 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
   const int kv_head = head / p.group;
   const int qw0 = q_block + wave * 16 * QB;
 
-  const uint16_t* qp = p.q + (int64_t)head * p.sq_h;
-  const uint16_t* kp = p.k + (int64_t)kv_head * p.sk_h;
-  const uint16_t* vp = p.v + (int64_t)kv_head * p.sv_h;
+  const uint16_t* qp = p.q + (int64_t)q0 * p.sq_t + (int64_t)head * p.sq_h;
+  const uint16_t* kp = p.k + (int64_t)k0 * p.sk_t + (int64_t)kv_head * p.sk_h;
+  const uint16_t* vp = p.v + (int64_t)k0 * p.sv_t + (int64_t)kv_head * p.sv_h;
 
   // The last key query i sees is causal_base + i (and no key past the chunk).
-  const int causal_base = p.q_local_offset + p.causal_shift - p.kv_local_offset;
+  const int causal_base = p.q_local_offset + causal_shift - p.kv_local_offset;
   // Keys at or beyond kv_end are invisible to every query of this workgroup;
   // those before wave_first are visible to every query of this wave.
-  int kv_end = p.kv_tokens;
-  int wave_first = p.kv_tokens;
+  int kv_end = kv_tokens;
+  int wave_first = kv_tokens;
   if (p.causal) {
-    kv_end = max(0, min(kv_end, causal_base + min(p.q_tokens, q_block + BLOCK_M)));
+    kv_end = max(0, min(kv_end, causal_base + min(q_tokens, q_block + BLOCK_M)));
     wave_first = min(wave_first, causal_base + qw0 + 1);
   }
   const int ntiles = (kv_end + kTileKeys - 1) / kTileKeys;
@@ -213,21 +227,26 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
   // the caller's buffers.
   // Wave-uniform byte address plus a 32-bit byte offset per lane: no vector
   // address arithmetic outside the edge tiles.
-  const int k_dma_d = 8 * Geo::k_granule((lane & 3) ^ (lane >> 4));
-  const int v_dma_d = 8 * ((lane & 3) ^ (2 * ((lane >> 4) & 1)));
-  const uint32_t k_dma_lane = 2u * ((lane >> 2) * (uint32_t)p.sk_t + k_dma_d);
-  const uint32_t v_dma_lane = VT ? 16u * lane : 2u * ((lane >> 2) * (uint32_t)p.sv_t + v_dma_d);
   auto dma = [](const uint16_t* base, uint32_t offset, uint8_t* dst) __attribute__((always_inline)) {
     asm volatile("" : "+s"(base));  // keeps the sum below uniform base + lane offset
     __builtin_amdgcn_global_load_lds((const SA_GLOBAL void*)(reinterpret_cast<const uint8_t*>(base) + offset),
                                      (SA_LDS void*)dst, 16, 0, 0);
   };
   auto issue_pieces = [&](int kt, uint8_t* stage, auto edge) __attribute__((always_inline)) {
+    // Where registers are short the lane offsets are worked out anew for each
+    // tile: held over the tile loop they cost head_dim 256 spills inside it
+    // (4.7 us per tile instead of 3.5).
+    int dma_lane = lane;
+    if constexpr (QB > 1 && DP >= 128) asm volatile("" : "+v"(dma_lane));
+    const int k_dma_d = 8 * Geo::k_granule((dma_lane & 3) ^ (dma_lane >> 4));
+    const int v_dma_d = 8 * ((dma_lane & 3) ^ (2 * ((dma_lane >> 4) & 1)));
+    const uint32_t k_dma_lane = 2u * ((dma_lane >> 2) * (uint32_t)p.sk_t + k_dma_d);
+    const uint32_t v_dma_lane = VT ? 16u * dma_lane : 2u * ((dma_lane >> 2) * (uint32_t)p.sv_t + v_dma_d);
     uint8_t* k_stage = stage;
     uint8_t* v_stage = stage + Geo::TILE_BYTES;
     const uint16_t* kt_base = kp + (int64_t)kt * p.sk_t;
     const uint16_t* vt_base = VT ? vp + (int64_t)kt * DP : vp + (int64_t)kt * p.sv_t;
-    const int last = p.kv_tokens - 1 - kt;  // last row of the chunk, in tile rows
+    const int last = kv_tokens - 1 - kt;  // last row of the chunk, in tile rows
 #pragma unroll
     for (int i = 0; i < Geo::PIECES / Geo::ISSUERS; ++i) {
       const int f = wave * (Geo::PIECES / Geo::ISSUERS) + i;
@@ -235,7 +254,7 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
       const int k_d0 = 32 * (f % CK);
       if constexpr (edge.value) {
         const int d = k_d0 + k_dma_d;
-        const uint32_t row = min(k_key0 + (lane >> 2), last);
+        const uint32_t row = min(k_key0 + (dma_lane >> 2), last);
         dma(kt_base, 2u * (row * (uint32_t)p.sk_t + (d < p.head_dim ? d : 0)), k_stage + f * 1024);
       } else {
         dma(kt_base + (int64_t)k_key0 * p.sk_t + k_d0, k_dma_lane, k_stage + f * 1024);
@@ -247,7 +266,7 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
         const int v_d0 = 32 * (f >> 2);
         if constexpr (edge.value) {
           const int d = v_d0 + v_dma_d;
-          const uint32_t row = min(v_key0 + (lane >> 2), last);
+          const uint32_t row = min(v_key0 + (dma_lane >> 2), last);
           dma(vt_base, 2u * (row * (uint32_t)p.sv_t + (d < p.head_dim ? d : 0)), v_stage + f * 1024);
         } else {
           dma(vt_base + (int64_t)v_key0 * p.sv_t + v_d0, v_dma_lane, v_stage + f * 1024);
@@ -257,7 +276,7 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
   };
   auto issue_tile = [&](int kt, uint8_t* stage) __attribute__((always_inline)) {
     if (wave >= Geo::ISSUERS) return;
-    if (kt + kTileKeys > p.kv_tokens || p.head_dim < DP)
+    if (kt + kTileKeys > kv_tokens || p.head_dim < DP)
       issue_pieces(kt, stage, std::true_type());
     else
       issue_pieces(kt, stage, std::false_type());
@@ -277,7 +296,7 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
     qi[qb] = qw0 + 16 * qb + r16;
-    const bool ok = qi[qb] < p.q_tokens;
+    const bool ok = qi[qb] < q_tokens;
 #pragma unroll
     for (int c = 0; c < CK; ++c) {
       const int d = 32 * c + 8 * j;
@@ -298,7 +317,7 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
     l_part[qb] = 0.f;
 #pragma unroll
     for (int db = 0; db < DB; ++db) acc[db][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (!p.init && qi[qb] < p.q_tokens) {
+    if (!p.init && qi[qb] < q_tokens) {
       const int64_t blk = state_block(qi[qb], head, p.q_heads);
       const int64_t srow = p.tiled_state ? blk * 16 + r16 : (int64_t)qi[qb] * p.ss_t + (int64_t)head * p.ss_h;
       m_run[qb] = p.m[srow];
@@ -378,7 +397,7 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               const int key = key0 + 16 * kb + 4 * j + i;
-              const bool ok = key < p.kv_tokens && (!p.causal || key <= causal_base + qi[qb]);
+              const bool ok = key < kv_tokens && (!p.causal || key <= causal_base + qi[qb]);
               s[kb][qb][i] = ok ? s[kb][qb][i] : -INFINITY;
             }
       }
@@ -533,7 +552,7 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
     const int col8 = (lane % Geo::I8_GR) * 16 < p.head_dim ? (lane % Geo::I8_GR) * 16 : 0;
     auto issue_i8 = [&](int kt, uint8_t* stg) {
       if (wave >= Geo::I8_DMAS) return;
-      const int row = min(kt + row8, p.kv_tokens - 1);
+      const int row = min(kt + row8, kv_tokens - 1);
       __builtin_amdgcn_global_load_lds((const SA_GLOBAL void*)(kp8 + (int64_t)row * p.sk_t + col8),
                                        (SA_LDS void*)(stg + wave * 1024), 16, 0, 0);
       __builtin_amdgcn_global_load_lds((const SA_GLOBAL void*)(vp8 + (int64_t)row * p.sv_t + col8),
@@ -547,7 +566,7 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
     const bool dequantizes = tid < Geo::I8_GRANULES;
     auto load_scales = [&](int kt) {
       if (!dequantizes) return;
-      const int key = min(kt + tid / Geo::I8_GR, p.kv_tokens - 1);
+      const int key = min(kt + tid / Geo::I8_GR, kv_tokens - 1);
       const int64_t group = (int64_t)((p.scale_offset + key) >> p.scale_shift);
       ksc = ksp[group * p.sks_g];
       vsc = vsp[group * p.svs_g];
@@ -620,15 +639,14 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
   // The epilogue's parameters are read from the kernel's argument memory
   // again: kept in scalar registers across the tile loop they displaced its
   // own (the scalar spills took vector registers).
-  const SA_CONSTANT UpdateParams* args = (const SA_CONSTANT UpdateParams*)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(args));
   const SA_CONSTANT UpdateParams& e = *args;
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
     const float l_full = full_l(l_part[qb]);
-    if (qi[qb] >= e.q_tokens) continue;
+    if (qi[qb] >= q_tokens) continue;
     if (e.out != nullptr) {
-      uint16_t* orow = e.out + (int64_t)qi[qb] * e.so_t + (int64_t)head * e.so_h + 4 * j;
+      uint16_t* orow = e.out + (int64_t)(q0 + qi[qb]) * e.so_t + (int64_t)head * e.so_h + 4 * j;
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
         if (16 * db + 4 * j < e.head_dim) {
@@ -642,7 +660,7 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
         }
       }
       if (e.lse != nullptr && j == 0)
-        e.lse[(int64_t)head * e.lse_sh + e.lse_off + qi[qb]] =
+        e.lse[(int64_t)head * e.lse_sh + e.lse_off + q0 + qi[qb]] =
             l_full > 0.f ? (m_run[qb] + log2f(l_full)) * 0.69314718055994530942f : -INFINITY;
       continue;
     }
@@ -665,11 +683,17 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
 template <typename Op, int DP, int QB, int MODE>
 hipError_t launch_kernel(UpdateParams p, hipStream_t stream) {
   constexpr int rows = Geometry<DP>::WAVES * 16 * QB;
-  p.q_blocks = (p.q_tokens + rows - 1) / rows;
-  p.xcd_run = (int32_t)(((int64_t)p.q_blocks * p.q_heads + 7) / 8);
-  p.deal_blocks = p.causal && p.q_heads % 8 != 0;
-  hipLaunchKernelGGL((update_kernel<Op, DP, QB, MODE>), dim3(8u * (unsigned)p.xcd_run), dim3(Geometry<DP>::THREADS),
-                     0, stream, p);
+  const bool several = p.segments > 1;
+  p.numbering = p.q_heads % 8 == 0 ? kHeadsPerXcd : p.causal || several ? kDealt : kRunsPerXcd;
+  const int heads = p.numbering == kHeadsPerXcd ? p.q_heads / 8 : p.q_heads;
+  p.slots = 0;
+  for (int s = 0; s < (several ? p.segments : 1); ++s) {
+    p.first[s] = p.slots;
+    p.slots += ((several ? p.segment[s].q_len : p.q_tokens) + rows - 1) / rows * heads;
+  }
+  p.xcd_run = (p.slots + 7) / 8;
+  const unsigned grid = p.numbering == kHeadsPerXcd ? 8u * p.slots : p.numbering == kDealt ? p.slots : 8u * p.xcd_run;
+  hipLaunchKernelGGL((update_kernel<Op, DP, QB, MODE>), dim3(grid), dim3(Geometry<DP>::THREADS), 0, stream, p);
   return hipGetLastError();
 }
 

@@ -60,9 +60,9 @@ class StreamingAttentionConfig:
     require_pinned: bool = True
     pin_output: bool = True
     enable_nvtx: bool = False
-    # HBM-resident inputs with head_dim 128 read V through a transposed copy
-    # in device scratch (kv_heads * 128 * kv_tokens * 2 bytes, outside the
-    # workspace budget).  None: no cap; 0: never; otherwise the largest
+    # HBM-resident inputs with head_dim 128 and many queries read V through a
+    # transposed copy in device scratch (kv_heads * 128 * kv_tokens * 2 bytes,
+    # outside the workspace budget).  None: no cap; 0: never; otherwise the largest
     # scratch the runner may allocate.  Without it V is read in place, with
     # bit-identical results.
     resident_scratch_limit_bytes: int | None = None

@@ -184,10 +184,11 @@ class CudaWorkspace:
         """HBM-resident runs with head_dim 128: device scratch for V
         transposed per K/V head, [kv_heads, 128, kv_tokens padded to a
         multiple of 64] 16-bit elements, which the update kernel reads with
-        half the LDS instructions.  Grown on demand and kept for later runs;
-        outside the planner's workspace budget, like the resident inputs.
+        half the LDS instructions (in segments of enough queries to repay the
+        copy).  Grown on demand and kept for later runs; outside the planner's
+        workspace budget, like the resident inputs.
 
-        Returns the scratch bytes the next run will use, 0 when it reads V in
+        Returns the scratch bytes the next run may use, 0 when it reads V in
         place instead: ``limit_bytes`` caps the scratch (0 disables it), and
         an allocation that fails for lack of device memory also leaves the
         run on the in-place path, which gives the same results bit for bit.

@@ -1,0 +1,54 @@
+"""Segments launched together give each segment's own bits.
+
+HBM-resident runs launch up to 32 segments at once, ordered by their keys;
+each must get the output and LSE of a run that has it alone: empty, one-row
+and ragged segments, more than one launch's worth, heads that are and are not
+a multiple of the XCDs, causal with queries that see no key.
+"""
+
+from __future__ import annotations
+
+import itertools
+import random
+
+import pytest
+import torch
+
+from seqattn import StreamingAttentionConfig, StreamingAttentionRunner, build_plan
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim,dtype,count", [
+    (8, 2, 128, torch.bfloat16, 40),
+    (16, 16, 64, torch.float16, 33),
+    (6, 3, 96, torch.bfloat16, 32),
+    (8, 8, 256, torch.bfloat16, 2),
+    (4, 1, 32, torch.float16, 5),
+])
+def test_segments_together_equal_each_alone(q_heads, kv_heads, head_dim, dtype, count, causal):
+    print(f"[gpu case] segments {count} heads={q_heads}/{kv_heads} d={head_dim} {dtype} causal={causal}", flush=True)
+    rng = random.Random(count)
+    q_lengths = [rng.choice([0, 1, 17, 128, 129, 300]) for _ in range(count)]
+    k_lengths = [n and rng.choice([1, 63, 64, 65, 200, 700]) for n in q_lengths]
+    q_lengths[0], k_lengths[0] = 400, 650
+    cu_q, cu_k = ([0, *itertools.accumulate(x)] for x in (q_lengths, k_lengths))
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    q, k, v = (torch.randn((n, h, head_dim), generator=gen, device="cuda").to(dtype)
+               for n, h in ((cu_q[-1], q_heads), (cu_k[-1], kv_heads), (cu_k[-1], kv_heads)))
+    config = StreamingAttentionConfig(backend="hip", q_chunk_tokens=256, kv_chunk_tokens=192)
+    plan = build_plan(q_heads=q_heads, kv_heads=kv_heads, head_dim=head_dim, dtype=dtype, device="cuda",
+                      max_q_tokens=cu_q[-1], max_kv_tokens=cu_k[-1], config=config)
+    runner = StreamingAttentionRunner(plan, config)
+    out, lse = runner(q, k, v, torch.tensor(cu_q), torch.tensor(cu_k), causal=causal, return_lse=True)
+    for s in range(count):
+        rows, keys = slice(cu_q[s], cu_q[s + 1]), slice(cu_k[s], cu_k[s + 1])
+        if q_lengths[s] == 0:
+            continue
+        alone, alone_lse = runner(q[rows], k[keys], v[keys], torch.tensor([0, q_lengths[s]]),
+                                  torch.tensor([0, k_lengths[s]]), causal=causal, return_lse=True)
+        assert torch.equal(out[rows], alone), s
+        assert torch.equal(lse[:, rows], alone_lse), s
+    torch.cuda.synchronize()
+    runner.close()
