@@ -143,13 +143,15 @@ int64_t tiles_of(int64_t keys) { return (std::max<int64_t>(0, keys) + kTileKeys 
 // that.  No launch ends before its longest block.  Over 60 drawn shapes the
 // choice was within 3% of the best variant's time on average.
 double variant_time(const UpdateVariant& v, const UpdateParams& p, bool overlapped) {
+  // The narrowest workgroups pack the query heads of a K/V head.
+  const int64_t group = v.rows == kVariants[0][0].rows ? p.group : 1;
   double longest = 0, shortest = 0, work = 0, n = 0;
   const auto add = [&](int64_t q_len, int64_t k_len, int64_t first_visible) {
-    const double blocks = (double)((q_len + v.rows - 1) / v.rows) * p.q_heads;
+    const double blocks = (double)((q_len * group + v.rows - 1) / v.rows) * (p.q_heads / group);
     // Tiles of the last and the first block.
     const double last = tiles_of(p.causal ? std::min(k_len, first_visible + q_len - 1) : k_len);
     const double first =
-        p.causal ? tiles_of(std::min(k_len, first_visible + std::min<int64_t>(v.rows, q_len) - 1)) : last;
+        p.causal ? tiles_of(std::min(k_len, first_visible + std::min<int64_t>(v.rows / group, q_len) - 1)) : last;
     longest = std::max(longest, last);
     shortest = n == 0 ? first : std::min(shortest, first);
     work += 0.5 * (first + last) * blocks;

@@ -97,6 +97,11 @@ struct UpdateParams {
   int32_t q_tokens, kv_tokens, group, head_dim, q_heads;
   int32_t q_local_offset, kv_local_offset, causal_shift;
   int32_t causal, init;
+  // With pack (128-query workgroups of grouped-query launches) a row of a
+  // workgroup is one (query, query head of the K/V head) pair, `group` pairs
+  // per query, and unit_heads the K/V heads; else a row is a query and
+  // unit_heads the query heads.
+  int32_t pack, unit_heads;
   int32_t numbering;      // Numbering
   int32_t slots;          // workgroups of the launch (of one XCD, for kHeadsPerXcd)
   int32_t xcd_run;        // kRunsPerXcd: ceil(slots / 8)

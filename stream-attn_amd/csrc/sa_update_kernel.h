@@ -2,6 +2,7 @@
 // included by the sources that compile one head-dim's variants.
 #pragma once
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -174,9 +175,12 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
     kv_tokens = __builtin_amdgcn_readfirstlane(args->segment[s].k_len);
     causal_shift = kv_tokens - q_tokens;
   }
-  const int q_blocks = (q_tokens + BLOCK_M - 1) / BLOCK_M;
+  // Queries of one unit head; unit head and its query block.
+  const bool pack = QB == 1 && p.pack;
+  const int rows = pack ? q_tokens * p.group : q_tokens;
+  const int q_blocks = (rows + BLOCK_M - 1) / BLOCK_M;
   const int head_slot = slot / q_blocks;
-  const int head = head_slot + (p.numbering == kHeadsPerXcd ? (b & 7) * (p.q_heads >> 3) : 0);
+  const int unit = head_slot + (p.numbering == kHeadsPerXcd ? (b & 7) * (p.unit_heads >> 3) : 0);
   const int in_head = slot - head_slot * q_blocks;
   const int q_block = (p.causal ? q_blocks - 1 - in_head : in_head) * BLOCK_M;
 
@@ -185,8 +189,16 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
   const int lane = tid & 63;
   const int r16 = lane & 15;  // query within a 16-query block; key / d row within a 16-row fragment
   const int j = lane >> 4;    // k-slot group
-  const int kv_head = head / p.group;
+  const int kv_head = pack ? unit : unit / p.group;
   const int qw0 = q_block + wave * 16 * QB;
+
+  // Row qw0 + 16 qb + r16 is query qi[qb] of query head `head` (with pack
+  // that of this lane's row).
+  const auto query_of = [&](int row) { return pack ? (int)((uint32_t)row / (uint32_t)p.group) : row; };
+  int qi[QB];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) qi[qb] = query_of(qw0 + 16 * qb + r16);
+  const int head = pack ? unit * p.group + (qw0 + r16 - qi[0] * p.group) : unit;
 
   const uint16_t* qp = p.q + (int64_t)q0 * p.sq_t + (int64_t)head * p.sq_h;
   const uint16_t* kp = p.k + (int64_t)k0 * p.sk_t + (int64_t)kv_head * p.sk_h;
@@ -194,13 +206,16 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
 
   // The last key query i sees is causal_base + i (and no key past the chunk).
   const int causal_base = p.q_local_offset + causal_shift - p.kv_local_offset;
-  // Keys at or beyond kv_end are invisible to every query of this workgroup;
-  // those before wave_first are visible to every query of this wave.
+  // Keys at or beyond kv_end are invisible to every query of this workgroup
+  // and at or beyond wave_end to every query of this wave (a wave without
+  // queries sees none); those before wave_first are visible to all of them.
   int kv_end = kv_tokens;
+  int wave_end = qw0 < rows ? kv_tokens : 0;
   int wave_first = kv_tokens;
   if (p.causal) {
-    kv_end = max(0, min(kv_end, causal_base + min(q_tokens, q_block + BLOCK_M)));
-    wave_first = min(wave_first, causal_base + qw0 + 1);
+    kv_end = max(0, min(kv_end, causal_base + query_of(min(rows, q_block + BLOCK_M) - 1) + 1));
+    wave_end = min(wave_end, causal_base + query_of(min(rows, qw0 + 16 * QB) - 1) + 1);
+    wave_first = min(wave_first, causal_base + query_of(qw0) + 1);
   }
   const int ntiles = (kv_end + kTileKeys - 1) / kTileKeys;
   // The scale is fused into the exponent's FMA and the max is taken on raw
@@ -292,10 +307,8 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
 
   // Q fragments: query qw0 + 16 qb + r16, d = 32 c + 8 j .. +7.
   u32x4 qf[QB][CK];
-  int qi[QB];
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
-    qi[qb] = qw0 + 16 * qb + r16;
     const bool ok = qi[qb] < q_tokens;
 #pragma unroll
     for (int c = 0; c < CK; ++c) {
@@ -319,10 +332,11 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
     for (int db = 0; db < DB; ++db) acc[db][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (!p.init && qi[qb] < q_tokens) {
       const int64_t blk = state_block(qi[qb], head, p.q_heads);
-      const int64_t srow = p.tiled_state ? blk * 16 + r16 : (int64_t)qi[qb] * p.ss_t + (int64_t)head * p.ss_h;
+      const int r = qi[qb] & 15;  // r16, unless packed
+      const int64_t srow = p.tiled_state ? blk * 16 + r : (int64_t)qi[qb] * p.ss_t + (int64_t)head * p.ss_h;
       m_run[qb] = p.m[srow];
       l_part[qb] = j == 0 ? p.l[srow] : 0.f;
-      const float* arow = p.tiled_state ? p.acc + blk * 16 * p.head_dim + 4 * lane
+      const float* arow = p.tiled_state ? p.acc + blk * 16 * p.head_dim + 4 * (16 * j + r)
                                         : p.acc + (int64_t)qi[qb] * p.sa_t + (int64_t)head * p.sa_h + 4 * j;
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
@@ -348,6 +362,7 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
     for (int sub = 0; sub < kTileKeys / kSubKeys; ++sub) {
       const int rb = sub * kSubKeys;
       const int key0 = kt + rb;
+      if (key0 >= wave_end) break;
 
       // S^T: two 16-key blocks x QB 16-query blocks, CK 32-wide d steps.
       f32x4 s[2][QB];
@@ -665,12 +680,13 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
       continue;
     }
     const int64_t blk = state_block(qi[qb], head, e.q_heads);
-    const int64_t srow = e.tiled_state ? blk * 16 + r16 : (int64_t)qi[qb] * e.ss_t + (int64_t)head * e.ss_h;
+    const int r = qi[qb] & 15;
+    const int64_t srow = e.tiled_state ? blk * 16 + r : (int64_t)qi[qb] * e.ss_t + (int64_t)head * e.ss_h;
     if (j == 0) {
       e.m[srow] = m_run[qb];
       e.l[srow] = l_full;
     }
-    float* arow = e.tiled_state ? e.acc + blk * 16 * e.head_dim + 4 * lane
+    float* arow = e.tiled_state ? e.acc + blk * 16 * e.head_dim + 4 * (16 * j + r)
                                 : e.acc + (int64_t)qi[qb] * e.sa_t + (int64_t)head * e.sa_h + 4 * j;
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
@@ -684,12 +700,18 @@ template <typename Op, int DP, int QB, int MODE>
 hipError_t launch_kernel(UpdateParams p, hipStream_t stream) {
   constexpr int rows = Geometry<DP>::WAVES * 16 * QB;
   const bool several = p.segments > 1;
-  p.numbering = p.q_heads % 8 == 0 ? kHeadsPerXcd : p.causal || several ? kDealt : kRunsPerXcd;
-  const int heads = p.numbering == kHeadsPerXcd ? p.q_heads / 8 : p.q_heads;
+  int64_t most_queries = several ? 0 : p.q_tokens;
+  for (int s = 0; several && s < p.segments; ++s) most_queries = std::max<int64_t>(most_queries, p.segment[s].q_len);
+  p.pack = QB == 1 && p.group > 1 && most_queries * p.group <= INT32_MAX;
+  p.unit_heads = p.pack ? p.q_heads / p.group : p.q_heads;
+  p.numbering = p.unit_heads % 8 == 0 ? kHeadsPerXcd : p.causal || several ? kDealt : kRunsPerXcd;
+  const int heads = p.numbering == kHeadsPerXcd ? p.unit_heads / 8 : p.unit_heads;
+  const int per_query = p.pack ? p.group : 1;
   p.slots = 0;
   for (int s = 0; s < (several ? p.segments : 1); ++s) {
     p.first[s] = p.slots;
-    p.slots += ((several ? p.segment[s].q_len : p.q_tokens) + rows - 1) / rows * heads;
+    const int64_t queries = several ? p.segment[s].q_len : p.q_tokens;
+    p.slots += (int32_t)((queries * per_query + rows - 1) / rows * heads);
   }
   p.xcd_run = (p.slots + 7) / 8;
   const unsigned grid = p.numbering == kHeadsPerXcd ? 8u * p.slots : p.numbering == kDealt ? p.slots : 8u * p.xcd_run;
