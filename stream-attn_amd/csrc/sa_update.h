@@ -155,7 +155,7 @@ constexpr int kMaxVariants = 3;
 constexpr UpdateVariant kVariants[kHeadDims][kMaxVariants] = {
     {{128, 605, 920}, {256, 930, 1550}, {0, 0, 0}},
     {{128, 800, 1245}, {256, 1245, 2070}, {0, 0, 0}},
-    {{128, 1250, 2040}, {256, 1905, 0}, {384, 2620, 0}},
+    {{128, 1265, 2025}, {256, 1915, 0}, {384, 2600, 0}},
     {{128, 2460, 0}, {256, 3505, 0}, {0, 0, 0}},
 };
 

@@ -133,10 +133,10 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
   // each) and VB d blocks of V, as many as the registers hold.  Measured per
   // 64-key tile with one workgroup on every CU: head_dim 256, 32 queries per
   // wave, 3.4 us with (2, 4) and 3.9 us with (2, 2); 16 queries 2.3 us with
-  // (4, 8).  head_dim 128, 16 and 32 queries: VB 4 is 1-3% faster than 2; 48
-  // queries have no registers left for it.
+  // (4, 8).  head_dim 128, 48 queries on a full chip: 2.45 us with VB 8, 2.50
+  // with 2.
   constexpr int KB = DP == 256 ? (QB == 1 ? 4 : 2) : CK;
-  constexpr int VB = DP == 256 ? (QB == 1 ? 8 : 4) : DP == 32 || QB == 3 ? 2 : 4;
+  constexpr int VB = DP == 256 ? (QB == 1 ? 8 : 4) : DP == 32 ? 2 : DP == 128 && QB > 1 ? 8 : 4;
   constexpr int BLOCK_M = Geo::WAVES * 16 * QB;
   static_assert(!QUANT || (Geo::I8_DMAS <= Geo::WAVES && Geo::I8_GRANULES <= Geo::THREADS), "INT8 staging");
 
@@ -404,7 +404,7 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
             }
       }
 
-      if (key0 + kSubKeys > wave_first) {
+      if (__builtin_expect(key0 + kSubKeys > wave_first, 0)) {
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -440,15 +440,16 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
       bool any = false;
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
-        psum[qb] = exps(qb, m_run[qb] == -INFINITY ? 0.f : -m_run[qb], pf[qb]);
-        // Every p <= 2^8 (no logit above m + 8) whenever the lane's sum is;
-        // a row without a maximum yet always takes the rescale path.
-        grow[qb] = !(psum[qb] <= 256.f) || m_run[qb] == -INFINITY;
+        // Every p <= 2^8 (no logit above m + 8) whenever the lane's sum is.
+        // Against m = -inf (no maximum yet) every p is inf, or NaN where the
+        // key is masked, so such a row always takes the rescale path.
+        psum[qb] = exps(qb, -m_run[qb], pf[qb]);
+        grow[qb] = !(psum[qb] <= 256.f);
         any = any || grow[qb];
       }
       // Rescale only when some logit of the wave may have left the [.., m + 8]
       // window; where m stays, the values computed above stand.
-      if (__ballot(any) != 0) {
+      if (__builtin_expect(__ballot(any) != 0, 0)) {
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
           // The query's own decision: one of its four lanes saw a partial sum
@@ -462,13 +463,15 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
           float full = fmaxf(a, __shfl_xor(a, 16));
           full = fmaxf(full, __shfl_xor(full, 32));
           const float m_new = (mine && full > m_run[qb] + kRescaleThreshold) ? full : m_run[qb];
-          if (m_new != m_run[qb]) {
-            const float alpha = __builtin_amdgcn_exp2f(m_run[qb] - m_new);
+          // Without a maximum yet masked keys weigh 0 and NaN stays NaN.
+          const bool none = m_new == -INFINITY;
+          if (m_new != m_run[qb] || none) {
+            const float alpha = none ? 1.f : __builtin_amdgcn_exp2f(m_run[qb] - m_new);
             l_part[qb] *= alpha;
 #pragma unroll
             for (int db = 0; db < DB; ++db) acc[db][qb] *= alpha;
             m_run[qb] = m_new;
-            psum[qb] = exps(qb, -m_new, pf[qb]);
+            psum[qb] = exps(qb, none ? 0.f : -m_new, pf[qb]);
           }
         }
       }
