@@ -146,27 +146,31 @@ class HipExecutorMixin:
         self._check_lse(lse, q.shape[0])
         native_stats = _native.PipelineStats()
         compute = workspace.compute_stream
-        with torch.cuda.device(self.plan.device):
-            caller = torch.cuda.current_stream()
-            longest_k = max((b - a for a, b in zip(k_bounds[:-1], k_bounds[1:])), default=0)
-            stats.resident_scratch_bytes = workspace.attach_resident_scratch(
-                longest_k, self.config.resident_scratch_limit_bytes
-            )
-            if caller != compute:
-                compute.wait_stream(caller)
-        with torch.cuda.device(self.plan.device), self._range("seqattn:run_resident"):
+        longest_k = max((b - a for a, b in zip(k_bounds[:-1], k_bounds[1:])), default=0)
+        stats.resident_scratch_bytes = workspace.attach_resident_scratch(
+            longest_k, self.config.resident_scratch_limit_bytes
+        )
+        # The usual caller is on the compute stream itself, and the native
+        # call selects the device by itself: no device or stream object is
+        # made then (about a third of a short call's host time).
+        compute_ptr = compute.cuda_stream
+        caller = None
+        if torch._C._cuda_getCurrentRawStream(q.device.index) != compute_ptr:
+            caller = torch.cuda.current_stream(q.device)
+            compute.wait_stream(caller)
+        with self._range("seqattn:run_resident"):
             status = _native.lib().sa_pipeline_run_resident(
                 workspace.handle,
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                 None if lse is None else lse.data_ptr(),
-                q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
-                out.stride(0), out.stride(1), 0 if lse is None else lse.stride(0),
+                *q.stride()[:2], *k.stride()[:2], *v.stride()[:2], *out.stride()[:2],
+                0 if lse is None else lse.stride(0),
                 _bounds_array(q_bounds), _bounds_array(k_bounds), len(q_bounds) - 1,
                 float(scale), int(bool(causal)),
-                compute.cuda_stream, ctypes.byref(native_stats),
+                compute_ptr, ctypes.byref(native_stats),
             )
         _native.check(status, "sa_pipeline_run_resident")
-        if caller != compute:
+        if caller is not None:
             caller.wait_stream(compute)
         _merge_stats(stats, native_stats)
         return out

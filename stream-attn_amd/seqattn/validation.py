@@ -8,7 +8,7 @@ import torch
 def _segment_bounds(name: str, cu: torch.Tensor, total: int) -> list[int]:
     if cu.device.type != "cpu" or cu.ndim != 1 or cu.numel() < 2:
         raise ValueError(f"{name} must be a one-dimensional CPU tensor")
-    bounds = cu.to(dtype=torch.int64).tolist()
+    bounds = (cu if cu.dtype in (torch.int32, torch.int64) else cu.to(dtype=torch.int64)).tolist()
     if bounds[0] != 0 or bounds[-1] != total:
         raise ValueError(f"{name} must span [0, {total}], got {bounds}")
     if any(b < a for a, b in zip(bounds[:-1], bounds[1:])):
