@@ -192,8 +192,12 @@ int choose_rows(const UpdateParams& p, int d, int mode, bool overlapped) {
   double best = -1.0;
   for (UpdateVariant v : kVariants[d]) {
     if (!v.rows) continue;
-    // The INT8 staging of head_dim 128 leaves LDS for one workgroup.
-    if (mode == kInt8 && d == 2) v.two = 0;
+    if (mode == kInt8) {
+      // Dequantizing a tile takes about 4 ns per padded d, and the staging of
+      // head_dim 128 leaves LDS for one workgroup.
+      v.one += 4 * (32 << d);
+      v.two = d == 2 ? 0 : v.two + 8 * (32 << d);
+    }
     const double t = variant_time(v, p, overlapped);
     // Ties go to the wider workgroup (less traffic).
     if (best < 0.0 || t <= best) best = t, rows = v.rows;
