@@ -22,7 +22,7 @@
 //
 // Streamed chunks of a Q block of at least 512 rows are applied by two
 // launches, one per half of the block's rows: the first on the compute
-// stream, the second on the pipeline's own `side` stream (default priority).
+// stream, the second on the pipelines' `side` stream (default priority).
 // A span forks `side` from the compute stream and joins it back, and a slot
 // is refilled only after both halves recorded their kv_free events.  The two
 // halves' launches run concurrently, so one launch's partial last round of
@@ -39,6 +39,8 @@
 #include <cstdio>
 #include <cstring>
 #include <functional>
+#include <map>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -201,6 +203,41 @@ void add_stats(sa_pipeline_stats* st, int64_t h2d, int64_t d2h, int64_t qc, int6
   st->max_resident_q_tokens = std::max(st->max_resident_q_tokens, resident);
 }
 
+// The second launch stream of every pipeline on a device: created with the
+// first of them, destroyed with the last.  HIP deals streams onto a few
+// hardware queues as they are created; with a stream per pipeline the third
+// runner's landed on a queue of the other streams, and its two launch streams
+// took turns (65,536 x 32 heads in head groups: 75 ms a run instead of 58).
+// Launches of different pipelines on it run in order, like their copies on
+// the shared copy streams; everything a launch waits for was enqueued before
+// it, so none can wait for another's later work.
+struct SideStream {
+  hipStream_t stream = nullptr;
+  int users = 0;
+};
+std::mutex g_side_mutex;
+std::map<int, SideStream> g_side_streams;
+
+// The device is current.
+hipError_t acquire_side(sa_pipeline* p) {
+  std::lock_guard<std::mutex> lock(g_side_mutex);
+  SideStream& side = g_side_streams[p->device];
+  if (side.users == 0) {
+    const hipError_t err = hipStreamCreateWithFlags(&side.stream, hipStreamNonBlocking);
+    if (err != hipSuccess) return err;
+  }
+  ++side.users;
+  p->side = side.stream;
+  return hipSuccess;
+}
+
+void release_side(sa_pipeline* p) {
+  std::lock_guard<std::mutex> lock(g_side_mutex);
+  SideStream& side = g_side_streams[p->device];
+  if (--side.users == 0) (void)hipStreamDestroy(side.stream);
+  p->side = nullptr;
+}
+
 // Teardown: failures here cannot be acted on, so their codes are dropped.
 void release(sa_pipeline* p) {
   if (p->h2d) (void)hipStreamSynchronize(p->h2d);
@@ -237,7 +274,7 @@ void release(sa_pipeline* p) {
     if (p->h2d) (void)hipStreamDestroy(p->h2d);
     if (p->d2h) (void)hipStreamDestroy(p->d2h);
   }
-  if (p->side) (void)hipStreamDestroy(p->side);
+  if (p->side) release_side(p);
 }
 
 // Make the H2D stream wait until ring slot `slot` is no longer read by any
@@ -1444,7 +1481,7 @@ int32_t sa_pipeline_create(sa_pipeline** out_pipeline, int32_t device, void* q_b
     if (err == hipSuccess) err = hipEventCreateWithFlags(&p->kv_free[i], flags);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&p->kv_free_side[i], flags);
   }
-  if (err == hipSuccess) err = hipStreamCreateWithFlags(&p->side, hipStreamNonBlocking);
+  if (err == hipSuccess) err = acquire_side(p);
   if (err == hipSuccess) err = hipEventCreateWithFlags(&p->fork, flags);
   if (err == hipSuccess) err = hipEventCreateWithFlags(&p->join, flags);
   for (int i = 0; i < num_output_buffers && err == hipSuccess; ++i) {
@@ -1555,7 +1592,7 @@ int32_t sa_pipeline_create_head_groups(sa_pipeline** out_pipeline, int32_t devic
     if (err == hipSuccess) err = hipStreamCreateWithFlags(&p->d2h, hipStreamNonBlocking);
   }
   const unsigned flags = hipEventDisableTiming;
-  if (err == hipSuccess) err = hipStreamCreateWithFlags(&p->side, hipStreamNonBlocking);
+  if (err == hipSuccess) err = acquire_side(p);
   if (err == hipSuccess) err = hipEventCreateWithFlags(&p->fork, flags);
   if (err == hipSuccess) err = hipEventCreateWithFlags(&p->join, flags);
   for (int i = 0; i < num_sets && err == hipSuccess; ++i) {
