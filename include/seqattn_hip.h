@@ -512,7 +512,7 @@ int32_t sa_pipeline_kernel_busy(sa_pipeline* pipeline, double* busy_ms, double* 
 
 /*
  * sa_run_resident_noalloc: attention over HBM-resident Q/K/V into a
- * caller-owned device output (and LSE), allocating nothing.  No counterpart
+ * caller-owned device output (and LSE), allocating no device memory.  No counterpart
  * in the reference: it is for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  It computes what sa_pipeline_run_resident computes for

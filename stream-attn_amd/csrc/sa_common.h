@@ -79,8 +79,11 @@ struct SegmentGroup {
 // its fragments then take half the LDS instructions.  Measured with head_dim
 // 128: 0.3-0.7% faster at 65,536 and more queries x query heads per K/V head,
 // no gain at 32,768, 2-8% slower at 8,192 and below, where it also cannot
-// join a launch with other segments.
-inline bool transposes_v(int64_t q_length, int64_t group) { return q_length * group >= 65536; }
+// join a launch with other segments.  V read in place needs a token stride in
+// [1, 2^24) (32-bit offsets within a tile); the copy reads any.
+inline bool transposes_v(int64_t q_length, int64_t group, int64_t sv_t) {
+  return q_length * group >= 65536 || sv_t <= 0 || sv_t >= (1 << 24);
+}
 }  // namespace sa
 
 // Kernel entry points shared between the kernel and pipeline translation units.

@@ -13,6 +13,7 @@
 #include <cmath>
 #include <cstdint>
 #include <mutex>
+#include <new>
 #include <vector>
 
 #include "sa_common.h"
@@ -588,7 +589,7 @@ int32_t sa_run_resident_noalloc(const void* q, const void* k, const void* v, voi
                                 const int64_t* cu_seqlens_q, const int64_t* cu_seqlens_k,
                                 int32_t num_segments, int32_t q_heads, int32_t kv_heads,
                                 int32_t head_dim, int32_t dtype, int32_t kv_chunk_tokens,
-                                double softmax_scale, int32_t causal, void* stream) {
+                                double softmax_scale, int32_t causal, void* stream) try {
   sa::clear_error();
   if (!q || !k || !v || !out || !cu_seqlens_q || !cu_seqlens_k || num_segments < 0) {
     sa::set_error("sa_run_resident_noalloc: null argument");
@@ -678,7 +679,7 @@ int32_t sa_run_resident_noalloc(const void* q, const void* k, const void* v, voi
     const int64_t q_start = cu_seqlens_q[s], k_start = cu_seqlens_k[s];
     const int64_t q_length = cu_seqlens_q[s + 1] - q_start, k_length = cu_seqlens_k[s + 1] - k_start;
     if (q_length == 0) continue;
-    if (!sa::transposes_v(q_length, q_heads / kv_heads) && together.add(q_start, q_length, k_start, k_length)) continue;
+    if (!sa::transposes_v(q_length, q_heads / kv_heads, stride_vt) && together.add(q_start, q_length, k_start, k_length)) continue;
     const int64_t t_pad = (k_length + 63) / 64 * 64;
     rc = sa::launch_transpose_v(vd + k_start * stride_vt * 2, stride_vt, stride_vh, (int32_t)k_length, kv_heads, 128,
                                 vt, t_pad, hs);
@@ -692,6 +693,9 @@ int32_t sa_run_resident_noalloc(const void* q, const void* k, const void* v, voi
                               together.segments.data(), (int32_t)together.segments.size()};
   return launch(vd + together.k0 * stride_vt * 2, stride_vt, stride_vh, together.q0, together.q_span(), together.k0,
                 together.k_span(), fused, false);
+} catch (const std::bad_alloc&) {  // the list of segments
+  sa::set_error("sa_run_resident_noalloc: out of host memory");
+  return SA_ERR_BAD_STATE;
 }
 
 int32_t sa_update_attention_state(const void* q, const void* k, const void* v, float* running_max,

@@ -39,7 +39,6 @@
 #include <cstdio>
 #include <cstring>
 #include <functional>
-#include <map>
 #include <mutex>
 #include <string>
 #include <utility>
@@ -215,11 +214,13 @@ struct SideStream {
   hipStream_t stream = nullptr;
   int users = 0;
 };
+constexpr int kSideDevices = 64;  // pipelines on a device past these have a stream each
 std::mutex g_side_mutex;
-std::map<int, SideStream> g_side_streams;
+SideStream g_side_streams[kSideDevices];
 
 // The device is current.
 hipError_t acquire_side(sa_pipeline* p) {
+  if (p->device < 0 || p->device >= kSideDevices) return hipStreamCreateWithFlags(&p->side, hipStreamNonBlocking);
   std::lock_guard<std::mutex> lock(g_side_mutex);
   SideStream& side = g_side_streams[p->device];
   if (side.users == 0) {
@@ -232,10 +233,13 @@ hipError_t acquire_side(sa_pipeline* p) {
 }
 
 void release_side(sa_pipeline* p) {
+  const hipStream_t stream = std::exchange(p->side, nullptr);
+  if (p->device < 0 || p->device >= kSideDevices) {
+    (void)hipStreamDestroy(stream);
+    return;
+  }
   std::lock_guard<std::mutex> lock(g_side_mutex);
-  SideStream& side = g_side_streams[p->device];
-  if (--side.users == 0) (void)hipStreamDestroy(side.stream);
-  p->side = nullptr;
+  if (--g_side_streams[p->device].users == 0) (void)hipStreamDestroy(stream);
 }
 
 // Teardown: failures here cannot be acted on, so their codes are dropped.
@@ -1765,7 +1769,7 @@ int32_t sa_pipeline_run_resident(sa_pipeline* p, const void* q, const void* k, c
                                  int64_t lse_stride_h, const int64_t* cu_seqlens_q,
                                  const int64_t* cu_seqlens_k, int32_t num_segments,
                                  double softmax_scale, int32_t causal, void* compute_stream,
-                                 sa_pipeline_stats* stats) {
+                                 sa_pipeline_stats* stats) try {
   sa::clear_error();
   if (!p || !q || !k || !v || !out || !cu_seqlens_q || !cu_seqlens_k || num_segments < 0) {
     sa::set_error("sa_pipeline_run_resident: null argument");
@@ -1821,7 +1825,7 @@ int32_t sa_pipeline_run_resident(sa_pipeline* p, const void* q, const void* k, c
       const int64_t t_pad = (k_length + 63) / 64 * 64;
       const int64_t vt_bytes = (int64_t)p->kv_heads * 128 * t_pad * 2;
       const bool vt = p->head_dim == 128 && p->vt_scratch != nullptr && vt_bytes <= p->vt_scratch_bytes &&
-                      t_pad < (1 << 24) && sa::transposes_v(q_length, p->q_heads / p->kv_heads);
+                      t_pad < (1 << 24) && sa::transposes_v(q_length, p->q_heads / p->kv_heads, stride_vt);
       if (vt || !together.add(q_start, q_length, k_start, k_length)) {
         int32_t rc = 0;
         if (vt) {
@@ -1883,6 +1887,9 @@ int32_t sa_pipeline_run_resident(sa_pipeline* p, const void* q, const void* k, c
     if (rc != 0) return rc;
   }
   return 0;
+} catch (const std::bad_alloc&) {  // the list of segments
+  sa::set_error("sa_pipeline_run_resident: out of host memory");
+  return SA_ERR_BAD_STATE;
 }
 
 int32_t sa_pipeline_finalize(sa_pipeline* p, int32_t slot, int32_t q_tokens, float* lse,

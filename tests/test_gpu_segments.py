@@ -8,13 +8,14 @@ a multiple of the XCDs, causal with queries that see no key.
 
 from __future__ import annotations
 
+import ctypes
 import itertools
 import random
 
 import pytest
 import torch
 
-from seqattn import StreamingAttentionConfig, StreamingAttentionRunner, build_plan
+from seqattn import StreamingAttentionConfig, StreamingAttentionRunner, build_plan, _native
 
 pytestmark = pytest.mark.gpu
 
@@ -52,3 +53,28 @@ def test_segments_together_equal_each_alone(q_heads, kv_heads, head_dim, dtype, 
         assert torch.equal(lse[:, rows], alone_lse), s
     torch.cuda.synchronize()
     runner.close()
+
+
+def test_broadcast_v_rows_are_read_through_the_transposed_copy():
+    """V with a token stride of 0 cannot be read in place: it takes the copy whatever the segment's size."""
+    print("[gpu case] segments V token stride 0", flush=True)
+    heads, kv_heads, n, d = 8, 2, 200, 128
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v = (torch.randn((t, h, d), generator=gen, device="cuda").to(torch.bfloat16)
+               for t, h in ((n, heads), (n, kv_heads), (1, kv_heads)))
+    bounds = (ctypes.c_int64 * 3)(0, 77, n)
+
+    def run(values):
+        out, lse = torch.empty_like(q), torch.empty((heads, n), device="cuda")
+        _native.check(_native.lib().sa_run_resident_noalloc(
+            q.data_ptr(), k.data_ptr(), values.data_ptr(), out.data_ptr(), lse.data_ptr(), *q.stride()[:2],
+            *k.stride()[:2], *values.stride()[:2], *out.stride()[:2], lse.stride(0), bounds, bounds, 2, heads, kv_heads,
+            d, _native.SA_DTYPE_BF16, 128, 0.09, 1, torch.cuda.current_stream().cuda_stream), "sa_run_resident_noalloc")
+        return out, lse
+
+    broadcast = v.expand(n, kv_heads, d)
+    assert broadcast.stride(0) == 0
+    results = run(broadcast), run(broadcast.contiguous())
+    torch.cuda.synchronize()
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
