@@ -305,20 +305,24 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
     if (ntiles > 0) issue_tile(0, lds_a);
   }
 
-  // Q fragments: query qw0 + 16 qb + r16, d = 32 c + 8 j .. +7.
+  // Q fragments: query qw0 + 16 qb + r16, d = 32 c + 8 j .. +7.  Rows and
+  // granules past the end read the last query's d = 0 and are zeroed: loads
+  // under a branch each waited for the one before.
   u32x4 qf[QB][CK];
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
-    const bool ok = qi[qb] < q_tokens;
+    const uint16_t* row = qp + (int64_t)min(qi[qb], q_tokens - 1) * p.sq_t;
 #pragma unroll
     for (int c = 0; c < CK; ++c) {
       const int d = 32 * c + 8 * j;
-      if (ok && d < p.head_dim)
-        qf[qb][c] = *reinterpret_cast<const u32x4*>(qp + (int64_t)qi[qb] * p.sq_t + d) ^ q_sign(p.scale_log2);
-      else
-        qf[qb][c] = u32x4{0, 0, 0, 0};
+      qf[qb][c] = *reinterpret_cast<const u32x4*>(row + (d < p.head_dim ? d : 0));
     }
   }
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+    for (int c = 0; c < CK; ++c)
+      qf[qb][c] = qi[qb] < q_tokens && 32 * c + 8 * j < p.head_dim ? qf[qb][c] ^ q_sign(p.scale_log2) : u32x4{0, 0, 0, 0};
 
   // Online-softmax state (base-2 domain); acc[db][qb] holds d = 16 db + 4 j
   // .. +3 of query qi[qb], l_part this lane's share of l.
