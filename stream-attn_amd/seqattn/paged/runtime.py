@@ -9,7 +9,8 @@ Same entry point, arguments, validation and stats as the reference's
   256-token pages mean one scan of all K/V per 256 queries);
 * K/V pages are gathered into ring chunks of the planner's ``kv_chunk_tokens``
   by the native pipeline (``sa_pipeline_stream_kv_gather``), one H2D copy per
-  page piece and one kernel launch per chunk, chunk boundaries aligned to
+  page piece (pages next to each other in the caller's tensors go together) and
+  one kernel launch per chunk, chunk boundaries aligned to
   multiples of the chunk within the segment as in tensor mode;
 * page data reaches the copy engines from page-locked memory with no host
   copy where possible: the DRAM cache's slots are page-locked (hits are copied
@@ -121,9 +122,11 @@ class _StageRing:
 class _Load:
     """One K/V page on its way into page-locked memory."""
 
-    __slots__ = ("page", "future", "k_address", "v_address", "owner", "commit_slot", "ks_address", "vs_address")
+    __slots__ = ("page", "future", "k_address", "v_address", "owner", "commit_slot", "ks_address", "vs_address",
+                 "region")
 
-    def __init__(self, page, future, k_address, v_address, owner, commit_slot=None, ks_address=0, vs_address=0):
+    def __init__(self, page, future, k_address, v_address, owner, commit_slot=None, ks_address=0, vs_address=0,
+                 region=None):
         self.page = page
         self.future = future
         self.k_address = k_address
@@ -132,6 +135,7 @@ class _Load:
         self.commit_slot = commit_slot
         self.ks_address = ks_address
         self.vs_address = vs_address
+        self.region = region
 
 
 class PagedAttentionRunner:
@@ -449,7 +453,7 @@ class PagedAttentionRunner:
             if load.commit_slot is not None:
                 state.cache.commit(load.page, load.commit_slot)
             queue.push(Fragment(load.k_address, load.v_address, load.page.valid_tokens, load.owner,
-                                load.ks_address, load.vs_address))
+                                load.ks_address, load.vs_address, load.region))
             stats.kv_pages += 1
             if queue.rows >= kv_chunk:
                 issue((queue.rows // kv_chunk) * kv_chunk)
@@ -637,7 +641,8 @@ class _RunState:
         if self.zero_copy_kv is not None:
             k_rows, v_rows = self.zero_copy_kv.pinned_kv_rows(page.token_start, page.token_stop)
             self.cache.lookup(page)
-            return _Load(page, None, k_rows.data_ptr(), v_rows.data_ptr(), None)
+            region = (k_rows.untyped_storage().data_ptr(), v_rows.untyped_storage().data_ptr())
+            return _Load(page, None, k_rows.data_ptr(), v_rows.data_ptr(), None, region=region)
         slot, lookup = self.cache.lookup(page)
         stats.cache_lookup_seconds += lookup.seconds
         record = self.cache.record(page) if self.cache.records else None

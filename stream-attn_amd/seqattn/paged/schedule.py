@@ -95,7 +95,8 @@ def plan_q_groups(pages: Sequence[PageDescriptor], block_rows: int) -> list[QGro
 class Fragment:
     """Contiguous host rows of K and V (addresses) plus the owner released
     once the rows have been copied; INT8 pages also carry per-row K and V
-    scale addresses."""
+    scale addresses.  Rows read in place name the page-locked allocations they
+    lie in (`region`)."""
 
     k_address: int
     v_address: int
@@ -103,11 +104,17 @@ class Fragment:
     owner: object = None
     ks_address: int = 0
     vs_address: int = 0
+    region: tuple[int, int] | None = None
 
 
 @dataclass
 class FragmentQueue:
-    """K/V rows waiting for their H2D copy, in segment order."""
+    """K/V rows waiting for their H2D copy, in segment order.
+
+    A fragment that continues the last one within the same allocations joins
+    it: one copy of a whole chunk instead of one per page (1 MB pages of 16,384
+    x 16 heads x d128: 128 copies of 24 us with 10-15 us between them).
+    """
 
     row_bytes: int
     scale_row_bytes: int = 0
@@ -115,9 +122,16 @@ class FragmentQueue:
     rows: int = 0
 
     def push(self, fragment: Fragment) -> None:
-        if fragment.rows > 0:
+        if fragment.rows <= 0:
+            return
+        self.rows += fragment.rows
+        last = self.fragments[-1] if self.fragments else None
+        if (last is not None and fragment.region is not None and fragment.region == last.region
+                and fragment.k_address == last.k_address + last.rows * self.row_bytes
+                and fragment.v_address == last.v_address + last.rows * self.row_bytes):
+            last.rows += fragment.rows
+        else:
             self.fragments.append(fragment)
-            self.rows += fragment.rows
 
     def take(self, rows: int) -> tuple[list[tuple[int, int, int, int, int]], list[object]]:
         """Remove the first ``rows`` rows: returns (k, v, rows, k_scales,

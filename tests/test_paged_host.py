@@ -266,6 +266,22 @@ def test_fragment_queue_advances_int8_scale_rows():
     assert pieces == [(2128, 6128, 2, 8008, 8508)]
 
 
+def test_fragment_queue_joins_neighbouring_rows_of_one_allocation_only():
+    queue = FragmentQueue(row_bytes=10)
+    region = (1000, 5000)
+    for k, v, rows, where in ((1000, 5000, 3, region), (1030, 5030, 2, region), (1050, 5050, 2, (1050, 5050)),
+                              (1070, 5070, 1, (1050, 5050)), (1080, 5090, 1, (1050, 5050)), (1090, 5100, 1, None),
+                              (1100, 5110, 1, None)):
+        queue.push(Fragment(k, v, rows, region=where))
+    pieces, done = queue.take(4)
+    assert pieces == [(1000, 5000, 4, 0, 0)] and done == []
+    queue.push(Fragment(1110, 5120, 1))
+    pieces, done = queue.take(8)
+    assert [p[:3] for p in pieces] == [(1040, 5040, 1), (1050, 5050, 3), (1080, 5090, 1), (1090, 5100, 1),
+                                       (1100, 5110, 1), (1110, 5120, 1)]
+    assert done == [None] * 6 and queue.rows == 0
+
+
 def test_int8_slots_carry_per_row_scales():
     from seqattn.paged.cache import expand_token_scales, token_scale_layout
     from seqattn.paged.layout import KVLayout, PageDescriptor
