@@ -206,7 +206,8 @@ int choose_rows(const UpdateParams& p, int d, int mode, bool overlapped) {
   return rows;
 }
 
-hipError_t launch_update_variant(const UpdateParams& p, int mode, int dtype, bool overlapped, hipStream_t stream) {
+hipError_t launch_update_variant(UpdateParams p, int mode, int dtype, bool overlapped, hipStream_t stream) {
+  p.cus = overlapped ? kCUs / 2 : kCUs;
   const int d = p.head_dim <= 32 ? 0 : p.head_dim <= 64 ? 1 : p.head_dim <= 128 ? 2 : 3;
   const int rows = choose_rows(p, d, mode, overlapped);
   switch (d) {

@@ -14,7 +14,8 @@
 // other issues.  Each K/V fragment read from LDS feeds QB MFMAs.
 // K/V stream through LDS in 64-key tiles, two stages: the tile after the one
 // being computed is fetched by global_load_lds_dwordx4 (HBM/L2 -> LDS with
-// no register staging) while the MFMAs run; one barrier per tile.
+// no register staging) while the MFMAs run; one barrier per tile.  Small
+// launches over many keys have four stages (three tiles in flight).
 //
 // v_mfma_f32_16x16x32_{bf16,f16}: A 16x32 (lane l: row l % 16, k 8 (l / 16)
 // .. +7), B 32x16 (lane l: column l % 16, k 8 (l / 16) .. +7), C 16x16 (lane
@@ -105,6 +106,7 @@ struct UpdateParams {
   int32_t numbering;      // Numbering
   int32_t slots;          // workgroups of the launch (of one XCD, for kHeadsPerXcd)
   int32_t xcd_run;        // kRunsPerXcd: ceil(slots / 8)
+  int32_t cus;            // CUs the launch has to itself (host only)
   float scale_log2;
   // INT8 K/V only: fp16 scales, element (group, kv_head) at
   // scales[group * s?s_g + kv_head * s?s_h], group = (scale_offset + key) >> scale_shift.

@@ -122,11 +122,15 @@ struct Geometry {
 // tile by tile, each 32-key group in the k-slot order of P^T (slot s holds
 // key 16 ((s >> 2) & 1) + 4 (s >> 3) + (s & 3)), zero keys up to a multiple
 // of 64.
-template <typename Op, int DP, int QB, int MODE>
+// STAGES: LDS stages, of which all but one are in flight while a tile is
+// computed (2, or a power of two above it for V read in place).
+template <typename Op, int DP, int QB, int MODE, int STAGES>
 __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const UpdateParams p) {
   using Geo = Geometry<DP>;
   constexpr bool VT = MODE == kTransposedV;
   constexpr bool QUANT = MODE == kInt8;
+  constexpr bool RING = STAGES > 2;
+  static_assert(!RING || (MODE == kRows && (STAGES & (STAGES - 1)) == 0), "ring of stages");
   constexpr int CK = Geo::CK;
   constexpr int DB = Geo::DB;
   // Fragments read before one wait: KB 32-wide d steps of K (two fragments
@@ -144,8 +148,12 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
   // below names one of them statically, so the compiler can tell that the
   // in-flight prefetch into one stage does not alias reads of the other and
   // need not wait for it.
-  __shared__ __attribute__((aligned(1024))) uint8_t lds_a[2 * Geo::TILE_BYTES];
-  __shared__ __attribute__((aligned(1024))) uint8_t lds_b[2 * Geo::TILE_BYTES];
+  // A ring of more stages is lds_a alone: its tiles are only read by inline
+  // asm, which the compiler does not relate to the DMA (no wait of its own
+  // stands in the loop).
+  constexpr int STAGE_BYTES = 2 * Geo::TILE_BYTES;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds_a[RING ? STAGES * STAGE_BYTES : STAGE_BYTES];
+  __shared__ __attribute__((aligned(1024))) uint8_t lds_b[RING ? 16 : STAGE_BYTES];
   // INT8 staging (K then V of one raw tile), also two distinct objects.
   constexpr int kStagingBytes = QUANT ? 2 * Geo::I8_TILE_BYTES : 16;
   __shared__ __attribute__((aligned(1024))) uint8_t lds_qa[kStagingBytes];
@@ -323,6 +331,11 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
 #pragma unroll
     for (int c = 0; c < CK; ++c)
       qf[qb][c] = qi[qb] < q_tokens && 32 * c + 8 * j < p.head_dim ? qf[qb][c] ^ q_sign(p.scale_log2) : u32x4{0, 0, 0, 0};
+
+  // The ring's other tiles, behind the wait for Q.
+  if constexpr (RING) {
+    for (int t = 1; t < min(ntiles, STAGES - 1); ++t) issue_tile(t * kTileKeys, lds_a + t * STAGE_BYTES);
+  }
 
   // Online-softmax state (base-2 domain); acc[db][qb] holds d = 16 db + 4 j
   // .. +3 of query qi[qb], l_part this lane's share of l.
@@ -536,9 +549,40 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
     return h + __shfl_xor(h, 32);
   };
 
-  if constexpr (!QUANT) {
+  int until_merge = p.merge_tiles;  // tiles left in the current K/V chunk
+  auto merge_after_tile = [&]() {
+    if (p.merge_tiles > 0 && --until_merge == 0) {
+      until_merge = p.merge_tiles;
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        const float full = full_l(l_part[qb]);
+        l_part[qb] = j == 0 ? full : 0.f;
+      }
+    }
+  };
+  if constexpr (RING) {
+    // As below, with tiles t+1 .. t+STAGES-2 in flight across the barrier.
+    // An issuing wave's DMA completes in order, PER_TILE of them per tile, so
+    // tile t is there once no more than the later tiles' are outstanding.
+    constexpr int PER_TILE = 2 * Geo::PIECES / Geo::ISSUERS;
+    static_assert((STAGES - 2) * PER_TILE <= 63, "vmcnt range");
+    static_assert(STAGES == 4, "waits below");
+    for (int t = 0; t < ntiles; ++t) {
+      const int later = ntiles - 1 - t;
+      if (later >= 2)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER_TILE) : "memory");
+      else if (later == 1)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER_TILE) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (later >= STAGES - 1)
+        issue_tile((t + STAGES - 1) * kTileKeys, lds_a + ((t + STAGES - 1) & (STAGES - 1)) * STAGE_BYTES);
+      compute(t, lds_a + (t & (STAGES - 1)) * STAGE_BYTES);
+      merge_after_tile();
+    }
+  } else if constexpr (!QUANT) {
     // Tile t is computed from `cur` while tile t+1 streams into `next`.
-    int until_merge = p.merge_tiles;  // tiles left in the current K/V chunk
     auto tile = [&](int t, const uint8_t* cur, uint8_t* next) {
       // Every wave waits for its own DMA of tile t before the barrier, so
       // after it all 64 rows of `cur` are in LDS.  LDS DMA is counted by
@@ -550,14 +594,7 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
       __syncthreads();
       if (t + 1 < ntiles) issue_tile((t + 1) * kTileKeys, next);
       compute(t, cur);
-      if (p.merge_tiles > 0 && --until_merge == 0) {
-        until_merge = p.merge_tiles;
-#pragma unroll
-        for (int qb = 0; qb < QB; ++qb) {
-          const float full = full_l(l_part[qb]);
-          l_part[qb] = j == 0 ? full : 0.f;
-        }
-      }
+      merge_after_tile();
     };
     for (int t = 0; t < ntiles; t += 2) {
       tile(t, lds_a, lds_b);
@@ -723,14 +760,32 @@ hipError_t launch_kernel(UpdateParams p, hipStream_t stream) {
   const int heads = p.numbering == kHeadsPerXcd ? p.unit_heads / 8 : p.unit_heads;
   const int per_query = p.pack ? p.group : 1;
   p.slots = 0;
+  [[maybe_unused]] int64_t keys = several ? 0 : p.kv_tokens;
   for (int s = 0; s < (several ? p.segments : 1); ++s) {
+    if (several) keys += p.segment[s].k_len;
     p.first[s] = p.slots;
     const int64_t queries = several ? p.segment[s].q_len : p.q_tokens;
     p.slots += (int32_t)((queries * per_query + rows - 1) / rows * heads);
   }
   p.xcd_run = (p.slots + 7) / 8;
   const unsigned grid = p.numbering == kHeadsPerXcd ? 8u * p.slots : p.numbering == kDealt ? p.slots : 8u * p.xcd_run;
-  hipLaunchKernelGGL((update_kernel<Op, DP, QB, MODE>), dim3(grid), dim3(Geometry<DP>::THREADS), 0, stream, p);
+  if constexpr (QB == 1 && MODE == kRows && DP <= 128) {
+    // Workgroups that have a CU to themselves have the LDS for two more tiles
+    // in flight, where two stages waited for HBM at every barrier (head_dim
+    // 128, 24 decoding sequences of 8,000 keys, 786 MB of K and V, 272 -> 235
+    // us; 1,009 queries over 61,312 keys, 251 MB, 1,137 -> 1,040 us).  K and V
+    // that the XCDs' L2 (4 MB each) hold come back soon enough, and two
+    // workgroups on a CU hide each other's waits: there the ring's longer
+    // start and loop took 5% (2,476 x 8 heads, 10 MB) and 2% (head_dim 64,
+    // 420 workgroups) more.
+    constexpr int64_t kL2Bytes = int64_t(8 * 4) << 20;
+    const int64_t workgroups = (int64_t)p.slots * (p.numbering == kHeadsPerXcd ? 8 : 1);
+    if (workgroups <= p.cus && 4 * keys * (p.q_heads / p.group) * p.head_dim > kL2Bytes) {
+      hipLaunchKernelGGL((update_kernel<Op, DP, QB, MODE, 4>), dim3(grid), dim3(Geometry<DP>::THREADS), 0, stream, p);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((update_kernel<Op, DP, QB, MODE, 2>), dim3(grid), dim3(Geometry<DP>::THREADS), 0, stream, p);
   return hipGetLastError();
 }
 
