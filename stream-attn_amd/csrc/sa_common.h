@@ -8,7 +8,7 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
-#include <string>
+#include <exception>
 #include <vector>
 
 #include "seqattn_hip.h"
@@ -17,6 +17,10 @@ namespace sa {
 
 void set_error(const char* fmt, ...);
 void clear_error();
+
+// The return code, and message, of an entry point that an exception reached
+// (host memory that a list or a callback could not get).
+int32_t exception_status(const char* entry_point, const std::exception& error);
 
 // Converts a hipError_t into the ABI convention (0 or a positive code) and
 // records a message naming the failing call.

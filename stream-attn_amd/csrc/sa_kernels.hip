@@ -694,9 +694,8 @@ int32_t sa_run_resident_noalloc(const void* q, const void* k, const void* v, voi
                               together.segments.data(), (int32_t)together.segments.size()};
   return launch(vd + together.k0 * stride_vt * 2, stride_vt, stride_vh, together.q0, together.q_span(), together.k0,
                 together.k_span(), fused, false);
-} catch (const std::bad_alloc&) {  // the list of segments
-  sa::set_error("sa_run_resident_noalloc: out of host memory");
-  return SA_ERR_BAD_STATE;
+} catch (const std::exception& error) {
+  return sa::exception_status("sa_run_resident_noalloc", error);
 }
 
 int32_t sa_update_attention_state(const void* q, const void* k, const void* v, float* running_max,

@@ -40,7 +40,6 @@
 #include <cstring>
 #include <functional>
 #include <mutex>
-#include <string>
 #include <utility>
 #include <vector>
 
@@ -49,19 +48,23 @@
 namespace sa {
 
 namespace {
-thread_local std::string g_last_error;
+thread_local char g_last_error[512] = "";  // needs no allocation, so reporting cannot fail
 }
 
 void set_error(const char* fmt, ...) {
-  char buf[512];
   va_list ap;
   va_start(ap, fmt);
-  vsnprintf(buf, sizeof(buf), fmt, ap);
+  vsnprintf(g_last_error, sizeof(g_last_error), fmt, ap);
   va_end(ap);
-  g_last_error = buf;
 }
 
-void clear_error() { g_last_error.clear(); }
+void clear_error() { g_last_error[0] = '\0'; }
+
+int32_t exception_status(const char* entry_point, const std::exception& error) {
+  const bool memory = dynamic_cast<const std::bad_alloc*>(&error) != nullptr;
+  set_error("%s: %s", entry_point, memory ? "out of host memory" : error.what());
+  return SA_ERR_BAD_STATE;
+}
 
 int32_t hip_status(hipError_t err, const char* what) {
   if (err == hipSuccess) return 0;
@@ -272,8 +275,10 @@ void release(sa_pipeline* p) {
     if (p->set_done[i]) (void)hipEventDestroy(p->set_done[i]);
     if (p->set_free[i]) (void)hipEventDestroy(p->set_free[i]);
   }
-  for (hipEvent_t e : p->t_start) (void)hipEventDestroy(e);
-  for (hipEvent_t e : p->t_stop) (void)hipEventDestroy(e);
+  for (hipEvent_t e : p->t_start)
+    if (e) (void)hipEventDestroy(e);
+  for (hipEvent_t e : p->t_stop)
+    if (e) (void)hipEventDestroy(e);
   if (p->owns_streams) {
     if (p->h2d) (void)hipStreamDestroy(p->h2d);
     if (p->d2h) (void)hipStreamDestroy(p->d2h);
@@ -306,6 +311,19 @@ int32_t load_q(sa_pipeline* p, const void* q_host, int32_t q_tokens, hipStream_t
   return 0;
 }
 
+// Records the start of the next timed launch (its stop is t_stop[t_used++]).
+int32_t start_timing(sa_pipeline* p, hipStream_t stream) {
+  if (p->t_used == p->t_stop.size()) {
+    // The events' places come first, so that none is lost.
+    p->t_start.resize(p->t_used + 1, nullptr);
+    p->t_stop.resize(p->t_used + 1, nullptr);
+  }
+  if (!p->t_start[p->t_used]) SA_HIP_RETURN(hipEventCreate(&p->t_start[p->t_used]));
+  if (!p->t_stop[p->t_used]) SA_HIP_RETURN(hipEventCreate(&p->t_stop[p->t_used]));
+  SA_HIP_RETURN(hipEventRecord(p->t_start[p->t_used], stream));
+  return 0;
+}
+
 // One update launch over rows [start, start + n) of a K/V span, optionally
 // bracketed by timing events.
 int32_t launch_timed(sa_pipeline* p, const void* q, int64_t sq_t, int64_t sq_h, const void* k,
@@ -316,16 +334,8 @@ int32_t launch_timed(sa_pipeline* p, const void* q, int64_t sq_t, int64_t sq_h, 
                      const sa::FusedOutput* fused = nullptr, int32_t state_row = 0,
                      bool v_transposed = false) {
   TraceRange range(p->trace, "seqattn:fused_update");
-  if (p->timing) {
-    if (p->t_used == p->t_start.size()) {
-      hipEvent_t a = nullptr, b = nullptr;
-      SA_HIP_RETURN(hipEventCreate(&a));
-      SA_HIP_RETURN(hipEventCreate(&b));
-      p->t_start.push_back(a);
-      p->t_stop.push_back(b);
-    }
-    SA_HIP_RETURN(hipEventRecord(p->t_start[p->t_used], compute));
-  }
+  if (p->timing)
+    if (const int32_t trc = start_timing(p, compute)) return trc;
   const int64_t qt = (int64_t)p->q_heads * p->head_dim;
   const int64_t srow = (int64_t)state_row * p->q_heads;
   int32_t rc = sa::launch_update(q, k, v, p->m + srow, p->l + srow, p->acc + srow * p->head_dim, sq_t,
@@ -345,16 +355,8 @@ int32_t launch_timed_int8(sa_pipeline* p, int slot, int32_t q_tokens, int32_t kv
                           int32_t q_local_offset, int32_t kv_local_offset, int32_t causal_shift,
                           double scale, int32_t flags, hipStream_t compute) {
   TraceRange range(p->trace, "seqattn:fused_update");
-  if (p->timing) {
-    if (p->t_used == p->t_start.size()) {
-      hipEvent_t a = nullptr, b = nullptr;
-      SA_HIP_RETURN(hipEventCreate(&a));
-      SA_HIP_RETURN(hipEventCreate(&b));
-      p->t_start.push_back(a);
-      p->t_stop.push_back(b);
-    }
-    SA_HIP_RETURN(hipEventRecord(p->t_start[p->t_used], compute));
-  }
+  if (p->timing)
+    if (const int32_t trc = start_timing(p, compute)) return trc;
   const int64_t qt = (int64_t)p->q_heads * p->head_dim;
   const int64_t kt = (int64_t)p->kv_heads * p->head_dim;
   int32_t rc = sa::launch_update_int8(
@@ -1015,16 +1017,8 @@ int32_t launch_unit(sa_pipeline* p, const void* q, int64_t sq_t, const void* k, 
                     int32_t kv_heads, int32_t causal_shift, double scale, int32_t causal, int32_t merge_keys,
                     const sa::FusedOutput& fused, bool v_transposed, bool overlapped, hipStream_t stream) {
   TraceRange range(p->trace, "seqattn:fused_update");
-  if (p->timing) {
-    if (p->t_used == p->t_start.size()) {
-      hipEvent_t a = nullptr, b = nullptr;
-      SA_HIP_RETURN(hipEventCreate(&a));
-      SA_HIP_RETURN(hipEventCreate(&b));
-      p->t_start.push_back(a);
-      p->t_stop.push_back(b);
-    }
-    SA_HIP_RETURN(hipEventRecord(p->t_start[p->t_used], stream));
-  }
+  if (p->timing)
+    if (const int32_t trc = start_timing(p, stream)) return trc;
   const int32_t flags =
       (causal ? SA_FLAG_CAUSAL : 0) | SA_FLAG_INITIALIZE | (overlapped ? sa::kLaunchOverlapped : 0);
   const int32_t rc = sa::launch_update(q, k, v, nullptr, nullptr, nullptr, sq_t, p->head_dim, sk_t, p->head_dim,
@@ -1385,7 +1379,7 @@ extern "C" {
 
 int32_t sa_abi_version(void) { return SA_ABI_VERSION; }
 
-const char* sa_last_error(void) { return sa::g_last_error.c_str(); }
+const char* sa_last_error(void) { return sa::g_last_error; }
 
 int32_t sa_pipeline_create(sa_pipeline** out_pipeline, int32_t device, void* q_buffer,
                            void* const* k_slots, void* const* v_slots, int32_t num_kv_buffers,
@@ -1393,7 +1387,7 @@ int32_t sa_pipeline_create(sa_pipeline** out_pipeline, int32_t device, void* q_b
                            void* const* out_slots, int32_t num_output_buffers,
                            int32_t q_chunk_tokens, int32_t kv_chunk_tokens, int32_t q_heads,
                            int32_t kv_heads, int32_t head_dim, int32_t dtype,
-                           void* h2d_stream, void* d2h_stream) {
+                           void* h2d_stream, void* d2h_stream) try {
   sa::clear_error();
   if (!out_pipeline) {
     sa::set_error("sa_pipeline_create: null out_pipeline");
@@ -1510,6 +1504,8 @@ int32_t sa_pipeline_create(sa_pipeline** out_pipeline, int32_t device, void* q_b
   }
   *out_pipeline = p;
   return 0;
+} catch (const std::exception& error) {
+  return sa::exception_status("sa_pipeline_create", error);
 }
 
 int32_t sa_pipeline_create_head_groups(sa_pipeline** out_pipeline, int32_t device, void* const* qo_sets,
@@ -1517,7 +1513,7 @@ int32_t sa_pipeline_create_head_groups(sa_pipeline** out_pipeline, int32_t devic
                                        int64_t vt_bytes, int32_t num_sets, int64_t max_q_tokens,
                                        int64_t max_kv_tokens, int32_t group_kv_heads, int32_t kv_chunk_tokens,
                                        int32_t q_heads, int32_t kv_heads, int32_t head_dim, int32_t dtype,
-                                       void* h2d_stream, void* d2h_stream) {
+                                       void* h2d_stream, void* d2h_stream) try {
   sa::clear_error();
   if (!out_pipeline) {
     sa::set_error("sa_pipeline_create_head_groups: null out_pipeline");
@@ -1612,6 +1608,8 @@ int32_t sa_pipeline_create_head_groups(sa_pipeline** out_pipeline, int32_t devic
   }
   *out_pipeline = p;
   return 0;
+} catch (const std::exception& error) {
+  return sa::exception_status("sa_pipeline_create_head_groups", error);
 }
 
 int32_t sa_pipeline_destroy(sa_pipeline* p) {
@@ -1638,7 +1636,7 @@ int32_t sa_pipeline_load_q(sa_pipeline* p, const void* q_host, int32_t q_tokens,
 int32_t sa_pipeline_stream_kv(sa_pipeline* p, const void* k_host, const void* v_host,
                               int32_t k_length, int32_t q_tokens, int32_t q_local_offset,
                               int32_t causal_shift, double softmax_scale, int32_t causal,
-                              void* compute_stream, sa_pipeline_stats* stats) {
+                              void* compute_stream, sa_pipeline_stats* stats) try {
   sa::clear_error();
   if (!p) return SA_ERR_INVALID_ARGUMENT;
   if (const int32_t hg = require_token_blocks(p, "sa_pipeline_stream_kv")) return hg;
@@ -1646,6 +1644,8 @@ int32_t sa_pipeline_stream_kv(sa_pipeline* p, const void* k_host, const void* v_
   SA_HIP_RETURN(guard.status());
   return stream_kv(p, k_host, v_host, k_length, q_tokens, q_local_offset, causal_shift,
                    softmax_scale, causal, static_cast<hipStream_t>(compute_stream), stats);
+} catch (const std::exception& error) {
+  return sa::exception_status("sa_pipeline_stream_kv", error);
 }
 
 int32_t sa_pipeline_stream_kv_span(sa_pipeline* p, const void* k_host, const void* v_host,
@@ -1653,7 +1653,7 @@ int32_t sa_pipeline_stream_kv_span(sa_pipeline* p, const void* k_host, const voi
                                    int32_t* initialize, int32_t q_tokens,
                                    int32_t q_local_offset, int32_t causal_shift,
                                    double softmax_scale, int32_t causal, void* compute_stream,
-                                   sa_pipeline_stats* stats) {
+                                   sa_pipeline_stats* stats) try {
   sa::clear_error();
   if (!p || !initialize || (kv_tokens > 0 && (!k_host || !v_host))) {
     sa::set_error("sa_pipeline_stream_kv_span: null argument");
@@ -1678,6 +1678,8 @@ int32_t sa_pipeline_stream_kv_span(sa_pipeline* p, const void* k_host, const voi
   }
   *initialize = init ? 1 : 0;
   return rc;
+} catch (const std::exception& error) {
+  return sa::exception_status("sa_pipeline_stream_kv_span", error);
 }
 
 int32_t sa_pipeline_stream_kv_gather(sa_pipeline* p, const void* const* k_fragments,
@@ -1686,7 +1688,7 @@ int32_t sa_pipeline_stream_kv_gather(sa_pipeline* p, const void* const* k_fragme
                                      int32_t kv_local_offset, int32_t* initialize,
                                      int32_t q_tokens, int32_t q_local_offset,
                                      int32_t causal_shift, double softmax_scale, int32_t causal,
-                                     void* compute_stream, sa_pipeline_stats* stats) {
+                                     void* compute_stream, sa_pipeline_stats* stats) try {
   sa::clear_error();
   if (!p || !initialize || num_fragments < 0 ||
       (num_fragments > 0 && (!k_fragments || !v_fragments || !fragment_tokens))) {
@@ -1703,6 +1705,8 @@ int32_t sa_pipeline_stream_kv_gather(sa_pipeline* p, const void* const* k_fragme
                             causal_shift, softmax_scale, causal, compute, stats);
   *initialize = init ? 1 : 0;
   return rc;
+} catch (const std::exception& error) {
+  return sa::exception_status("sa_pipeline_stream_kv_gather", error);
 }
 
 int32_t sa_pipeline_attach_int8_scales(sa_pipeline* p, void* const* k_scale_slots,
@@ -1739,7 +1743,7 @@ int32_t sa_pipeline_stream_kv_gather_int8(
     const void* const* k_scale_fragments, const void* const* v_scale_fragments,
     const int32_t* fragment_tokens, int32_t num_fragments, int32_t kv_local_offset,
     int32_t* initialize, int32_t q_tokens, int32_t q_local_offset, int32_t causal_shift,
-    double softmax_scale, int32_t causal, void* compute_stream, sa_pipeline_stats* stats) {
+    double softmax_scale, int32_t causal, void* compute_stream, sa_pipeline_stats* stats) try {
   sa::clear_error();
   if (!p || !initialize || num_fragments < 0 ||
       (num_fragments > 0 && (!k_fragments || !v_fragments || !k_scale_fragments ||
@@ -1760,6 +1764,8 @@ int32_t sa_pipeline_stream_kv_gather_int8(
                             causal_shift, softmax_scale, causal, compute, stats);
   *initialize = init ? 1 : 0;
   return rc;
+} catch (const std::exception& error) {
+  return sa::exception_status("sa_pipeline_stream_kv_gather_int8", error);
 }
 
 int32_t sa_pipeline_run_resident(sa_pipeline* p, const void* q, const void* k, const void* v,
@@ -1887,9 +1893,8 @@ int32_t sa_pipeline_run_resident(sa_pipeline* p, const void* q, const void* k, c
     if (rc != 0) return rc;
   }
   return 0;
-} catch (const std::bad_alloc&) {  // the list of segments
-  sa::set_error("sa_pipeline_run_resident: out of host memory");
-  return SA_ERR_BAD_STATE;
+} catch (const std::exception& error) {
+  return sa::exception_status("sa_pipeline_run_resident", error);
 }
 
 int32_t sa_pipeline_finalize(sa_pipeline* p, int32_t slot, int32_t q_tokens, float* lse,
@@ -2006,7 +2011,7 @@ int32_t sa_pipeline_set_kernel_timing(sa_pipeline* p, int32_t enable) {
   return 0;
 }
 
-int32_t sa_pipeline_kernel_busy(sa_pipeline* p, double* busy_ms, double* total_ms, int64_t* launches) {
+int32_t sa_pipeline_kernel_busy(sa_pipeline* p, double* busy_ms, double* total_ms, int64_t* launches) try {
   sa::clear_error();
   if (!p || !busy_ms || !total_ms || !launches) return SA_ERR_INVALID_ARGUMENT;
   sa::DeviceGuard guard(p->device);
@@ -2041,6 +2046,8 @@ int32_t sa_pipeline_kernel_busy(sa_pipeline* p, double* busy_ms, double* total_m
   *launches = (int64_t)p->t_used;
   p->t_used = 0;
   return 0;
+} catch (const std::exception& error) {
+  return sa::exception_status("sa_pipeline_kernel_busy", error);
 }
 
 int32_t sa_pipeline_kernel_timing(sa_pipeline* p, double* total_ms, int64_t* launches) {
@@ -2084,11 +2091,15 @@ int32_t sa_pipeline_run_device_output(sa_pipeline* p, const void* q_host, const 
   }
   sa::DeviceGuard guard(p->device);
   SA_HIP_RETURN(guard.status());
-  const int32_t rc = run_head_groups(p, static_cast<const char*>(q_host), static_cast<const char*>(k_host),
-                                     static_cast<const char*>(v_host), nullptr, lse, lse_stride_h, cu_seqlens_q,
-                                     cu_seqlens_k, num_segments, softmax_scale, causal,
-                                     static_cast<hipStream_t>(compute_stream), stats, static_cast<char*>(out),
-                                     stride_ot, stride_oh);
+  int32_t rc;
+  try {
+    rc = run_head_groups(p, static_cast<const char*>(q_host), static_cast<const char*>(k_host),
+                         static_cast<const char*>(v_host), nullptr, lse, lse_stride_h, cu_seqlens_q, cu_seqlens_k,
+                         num_segments, softmax_scale, causal, static_cast<hipStream_t>(compute_stream), stats,
+                         static_cast<char*>(out), stride_ot, stride_oh);
+  } catch (const std::exception& error) {
+    rc = sa::exception_status("sa_pipeline_run_device_output", error);
+  }
   if (rc != 0) drain_after_error(p);
   return rc;
 }
@@ -2106,8 +2117,13 @@ int32_t sa_pipeline_run(sa_pipeline* p, const void* q_host, const void* k_host, 
   }
   sa::DeviceGuard guard(p->device);
   SA_HIP_RETURN(guard.status());
-  const int32_t rc = run_host_output(p, q_host, k_host, v_host, out_host, lse, lse_stride_h, cu_seqlens_q,
-                                     cu_seqlens_k, num_segments, softmax_scale, causal, compute_stream, stats);
+  int32_t rc;
+  try {
+    rc = run_host_output(p, q_host, k_host, v_host, out_host, lse, lse_stride_h, cu_seqlens_q, cu_seqlens_k,
+                         num_segments, softmax_scale, causal, compute_stream, stats);
+  } catch (const std::exception& error) {
+    rc = sa::exception_status("sa_pipeline_run", error);
+  }
   if (rc != 0) drain_after_error(p);
   return rc;
 }

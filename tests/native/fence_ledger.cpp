@@ -18,16 +18,20 @@
 // ordering mistake the check must report.  ledger_fail_copy(n) makes the n-th
 // copy call fail (nothing is recorded for it): an error in the middle of a
 // run, after which ledger_unfinished() counts the copies and host functions
-// that were not complete when the call returned.
+// that were not complete when the call returned.  ledger_fail_allocation(n)
+// makes the pipeline's n-th allocation of host memory from then on throw (the
+// ledger's own are not counted).
 
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstdint>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <memory>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -65,6 +69,17 @@ struct Ledger {
 };
 
 Ledger g;
+
+// Allocations since ledger_fail_allocation, the one to fail (-1: none), and
+// how deep the ledger's own code is nested.
+long g_allocations = 0;
+long g_fail_allocation = -1;
+int g_recording = 0;
+
+struct Recording {
+  Recording() { ++g_recording; }
+  ~Recording() { --g_recording; }
+};
 
 // Whether this copy call is the one planted to fail.
 bool copy_fails() { return g.copies_seen++ == g.fail_copy; }
@@ -147,6 +162,16 @@ void lse_ranges(std::vector<Range>& out, const float* lse, int64_t sh, int64_t o
 
 }  // namespace
 
+// The library is linked so that its own allocations come here.
+void* operator new(size_t bytes) {
+  if (g_recording == 0 && g_allocations++ == g_fail_allocation) throw std::bad_alloc();
+  void* p = std::malloc(bytes ? bytes : 1);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+
 // --------------------------------------------------------------- HIP stubs
 const char* hipGetErrorString(hipError_t) { return "stub"; }
 hipError_t hipGetDevice(int* device) {
@@ -155,15 +180,18 @@ hipError_t hipGetDevice(int* device) {
 }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* stream, unsigned int) {
+  Recording own;
   *stream = new_handle<hipStream_t>();
   return hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t stream) {
+  Recording own;
   push(Op{kStreamSync, stream_id(stream), -1, {}, {}, "stream sync"});
   return hipSuccess;
 }
 hipError_t hipStreamWaitEvent(hipStream_t stream, hipEvent_t event, unsigned int) {
+  Recording own;
   const long n = g.waits_seen++;
   if (n == g.drop_wait) {
     ++g.dropped;
@@ -174,16 +202,19 @@ hipError_t hipStreamWaitEvent(hipStream_t stream, hipEvent_t event, unsigned int
   return hipSuccess;
 }
 hipError_t hipEventCreate(hipEvent_t* event) {
+  Recording own;
   *event = new_handle<hipEvent_t>();
   return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t* event, unsigned int) { return hipEventCreate(event); }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t event, hipStream_t stream) {
+  Recording own;
   g.last_record[event] = push(Op{kRecord, stream_id(stream), -1, {}, {}, "record"});
   return hipSuccess;
 }
 hipError_t hipEventSynchronize(hipEvent_t event) {
+  Recording own;
   auto it = g.last_record.find(event);
   push(Op{kEventSync, -1, it == g.last_record.end() ? -1 : it->second, {}, {}, "event sync"});
   return hipSuccess;
@@ -193,6 +224,7 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
   return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t stream) {
+  Recording own;
   if (copy_fails()) return hipErrorInvalidValue;
   const Kind k = kind == hipMemcpyHostToDevice ? kCopyH2D : kind == hipMemcpyDeviceToHost ? kCopyD2H : kCopyD2D;
   push(Op{k, stream_id(stream), -1, {span(src, (int64_t)bytes)}, {span(dst, (int64_t)bytes)},
@@ -203,6 +235,7 @@ hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKin
 // A strided copy reads and writes rows of `width` bytes on each side.
 hipError_t hipMemcpy2DAsync(void* dst, size_t dpitch, const void* src, size_t spitch, size_t width, size_t height,
                             hipMemcpyKind kind, hipStream_t stream) {
+  Recording own;
   if (copy_fails()) return hipErrorInvalidValue;
   const Kind k = kind == hipMemcpyHostToDevice ? kCopyH2D : kind == hipMemcpyDeviceToHost ? kCopyD2H : kCopyD2D;
   push(Op{k, stream_id(stream), -1, {strided(src, (int64_t)width, (int64_t)spitch, (int64_t)height)},
@@ -214,6 +247,7 @@ hipError_t hipMemcpy2DAsync(void* dst, size_t dpitch, const void* src, size_t sp
 // A host function is an operation of its stream with no device ranges; it
 // runs here at once (the tests that enqueue one give it real host memory).
 hipError_t hipLaunchHostFunc(hipStream_t stream, hipHostFn_t fn, void* user_data) {
+  Recording own;
   push(Op{kKernel, stream_id(stream), -1, {}, {}, "host function"});
   fn(user_data);
   return hipSuccess;
@@ -233,6 +267,7 @@ int32_t launch_update(const void* q, const void* k, const void* v, float* m, flo
                       int64_t sa_t, int64_t, int32_t q_tokens, int32_t kv_tokens, int32_t q_heads,
                       int32_t kv_heads, int32_t head_dim, int32_t, int32_t, int32_t, double, int32_t flags, int32_t,
                       hipStream_t stream, int32_t, const FusedOutput* fused, bool v_transposed, bool tiled) {
+  Recording own;
   Op op{kKernel, stream_id(stream), -1, {}, {}, "update"};
   op.reads.push_back(rows_of(q, q_tokens, sq_t, 2));
   op.reads.push_back(rows_of(k, kv_tokens, sk_t, 2));
@@ -260,6 +295,7 @@ int32_t launch_update(const void* q, const void* k, const void* v, float* m, flo
 
 int32_t launch_transpose_v(const void* v, int64_t sv_t, int64_t, int32_t kv_tokens, int32_t kv_heads, int32_t,
                            void* vt, int64_t t_pad, hipStream_t stream) {
+  Recording own;
   push(Op{kKernel, stream_id(stream), -1, {rows_of(v, kv_tokens, sv_t, 2)}, {span(vt, kv_heads * 128 * t_pad * 2)},
           "transpose v"});
   return 0;
@@ -271,6 +307,7 @@ int32_t launch_update_int8(const void* q, const void* k, const void* v, const vo
                            int64_t, int64_t sa_t, int64_t, int32_t q_tokens, int32_t kv_tokens, int32_t,
                            int32_t, int32_t, int32_t, int32_t, int32_t, int32_t, double, int32_t flags, int32_t,
                            int32_t, hipStream_t stream, bool tiled) {
+  Recording own;
   Op op{kKernel, stream_id(stream), -1, {}, {}, "update int8"};
   op.reads = {rows_of(q, q_tokens, sq_t, 2), rows_of(k, kv_tokens, sk_t, 1), rows_of(v, kv_tokens, sv_t, 1),
               rows_of(k_scales, kv_tokens, sks_g, 2), rows_of(v_scales, kv_tokens, svs_g, 2)};
@@ -285,6 +322,7 @@ int32_t launch_update_int8(const void* q, const void* k, const void* v, const vo
 int32_t launch_finalize(const float* acc, const float* m, const float* l, void* out, float* lse, int64_t sa_t,
                         int64_t, int64_t ss_t, int64_t, int64_t so_t, int64_t, int64_t lse_sh, int64_t lse_off,
                         int32_t q_tokens, int32_t q_heads, int32_t, int32_t, hipStream_t stream, bool tiled) {
+  Recording own;
   Op op{kKernel, stream_id(stream), -1, {}, {}, "finalize"};
   const int64_t rows = state_rows(q_tokens, tiled);
   op.reads = {rows_of(acc, rows, sa_t, 4), rows_of(m, rows, ss_t, 4), rows_of(l, rows, ss_t, 4)};
@@ -300,6 +338,7 @@ int32_t launch_finalize(const float* acc, const float* m, const float* l, void* 
 extern "C" {
 
 void ledger_reset(void) {
+  Recording own;
   g.ops.clear();
   g.last_record.clear();
   g.waits_seen = 0;
@@ -307,11 +346,19 @@ void ledger_reset(void) {
   g.dropped = 0;
   g.copies_seen = 0;
   g.fail_copy = -1;
+  g_fail_allocation = -1;
 }
 
 void ledger_drop_wait(long n) { g.drop_wait = n; }
 
 void ledger_fail_copy(long n) { g.fail_copy = n; }
+
+void ledger_fail_allocation(long n) {
+  g_allocations = 0;
+  g_fail_allocation = n;
+}
+
+long ledger_allocations(void) { return g_allocations; }
 
 long ledger_copies(void) { return g.copies_seen; }
 
@@ -321,6 +368,7 @@ long ledger_dropped(void) { return g.dropped; }
 
 // Counts of recorded operations: [copies H2D, copies D2H, kernels, waits].
 void ledger_counts(int64_t* out) {
+  Recording own;
   out[0] = out[1] = out[2] = out[3] = 0;
   for (const Op& op : g.ops) {
     if (op.kind == kCopyH2D) ++out[0];
@@ -333,6 +381,7 @@ void ledger_counts(int64_t* out) {
 // Returns the number of unordered conflicting pairs plus D2H copies not
 // complete at the last host synchronization; describes the first few in msg.
 int64_t ledger_check(char* msg, int64_t msg_len) {
+  Recording own;
   const int n = (int)g.ops.size();
   const int words = (n + 63) / 64;
   std::vector<uint64_t> reach((size_t)n * words, 0);  // reach[j] holds i when i happens before j
@@ -396,6 +445,7 @@ int64_t ledger_check(char* msg, int64_t msg_len) {
 // Copies and host functions (they touch host memory) not ordered before the
 // last host synchronization recorded so far.
 int64_t ledger_unfinished(void) {
+  Recording own;
   const int n = (int)g.ops.size();
   int last_sync = -1;
   for (int j = 0; j < n; ++j)

@@ -38,7 +38,7 @@ def ledger(tmp_path_factory):
     if compiler is None:
         pytest.skip("g++ is not available")
     out = tmp_path_factory.mktemp("ledger") / "libfence_ledger.so"
-    cmd = [compiler, "-shared", "-fPIC", "-std=c++17", "-O1", f"-I{ROOT / 'tests' / 'native' / 'hip_stub'}",
+    cmd = [compiler, "-shared", "-fPIC", "-std=c++17", "-O1", "-Wl,-Bsymbolic", f"-I{ROOT / 'tests' / 'native' / 'hip_stub'}",
            f"-I{ROOT / 'include'}", f"-I{ROOT / 'stream-attn_amd' / 'csrc'}",
            str(ROOT / "stream-attn_amd" / "csrc" / "sa_pipeline.cpp"), str(ROOT / "tests" / "native" / "fence_ledger.cpp"),
            "-o", str(out)]
@@ -56,6 +56,8 @@ def ledger(tmp_path_factory):
     lib.ledger_counts.argtypes = [ctypes.POINTER(ctypes.c_int64)]
     lib.ledger_fail_copy.argtypes = [ctypes.c_long]
     lib.ledger_copies.restype = ctypes.c_long
+    lib.ledger_fail_allocation.argtypes = [ctypes.c_long]
+    lib.ledger_allocations.restype = ctypes.c_long
     lib.ledger_unfinished.restype = ctypes.c_int64
     return lib
 
@@ -579,3 +581,129 @@ def test_a_failed_head_group_run_returns_with_its_copies_drained(ledger, num_set
 
     _failing_runs(ledger, run, f"head groups, sets={num_sets}, device output={device_output}")
 
+
+
+def _fail_each_allocation(ledger, run, label):
+    """Make each host allocation of a run fail in turn: the call reports it
+    and no copy it enqueued is still running when it returns."""
+    ledger.ledger_reset()
+    ledger.ledger_fail_allocation(-1)
+    status, unfinished, _ = run()
+    assert status == 0 and unfinished == 0, label
+    allocations = ledger.ledger_allocations()
+    assert allocations > 0, label
+    for n in range(allocations):
+        ledger.ledger_reset()
+        ledger.ledger_fail_allocation(n)
+        status, unfinished, message = run()
+        assert status == -4, f"{label}: allocation {n}"  # SA_ERR_BAD_STATE
+        assert b"out of host memory" in message, label
+        assert unfinished == 0, f"{label}: allocation {n}, {unfinished} copies in flight at the return"
+
+
+# Two output slots without timing allocate no host memory.
+@pytest.mark.parametrize("num_out,out_slots,timing", [(1, True, 0), (1, True, 1), (2, True, 1), (1, False, 0),
+                                                      (1, False, 1)])
+def test_out_of_host_memory_is_a_return_code_in_tensor_mode(ledger, num_out, out_slots, timing):
+    host = Space(0x5000_0000_0000)
+    cu_q, q_b = bounds([3000, 700])
+    cu_k, k_b = bounds([600, 300])
+
+    def run():
+        p = Pipeline(ledger, q_chunk=1024, kv_chunk=256, q_heads=4, kv_heads=2, head_dim=64, num_kv=2,
+                     num_out=num_out, out_slots=out_slots)
+        assert ledger.sa_pipeline_set_kernel_timing(p.handle, timing) == 0
+        q_host, k_host = host.take(q_b[-1] * p.q_row), host.take(k_b[-1] * p.kv_row)
+        v_host, out_host = host.take(k_b[-1] * p.kv_row), host.take(q_b[-1] * p.q_row)
+        status = ledger.sa_pipeline_run(p.handle, q_host, k_host, v_host, out_host, None, 0, cu_q, cu_k, 2, 0.125, 0,
+                                        p.compute, None)
+        unfinished = ledger.ledger_unfinished()
+        if status == 0 and timing:
+            busy, total, launches = ctypes.c_double(), ctypes.c_double(), ctypes.c_int64()
+            status = ledger.sa_pipeline_kernel_busy(p.handle, ctypes.byref(busy), ctypes.byref(total),
+                                                    ctypes.byref(launches))
+        message = ledger.sa_last_error()
+        p.destroy()
+        return status, unfinished, message
+
+    _fail_each_allocation(ledger, run, f"tensor mode, {num_out} output slots {out_slots}, timing {timing}")
+
+
+@pytest.mark.parametrize("device_output", [False, True])
+def test_out_of_host_memory_is_a_return_code_in_head_group_runs(ledger, device_output):
+    q_heads, kv_heads, head_dim = 4, 4, 64
+    dev = Space(0x7000_0000_0000)
+    host = Space(0x5000_0000_0000)
+    cu_q, q_b = bounds([1500, 900])
+    cu_k, k_b = bounds([1200, 900])
+    tq, tk = q_b[-1], k_b[-1]
+    row = q_heads * head_dim * HEAD_BYTES
+
+    def run():
+        sets = [(ctypes.c_void_p * 2)(*[dev.take(n * head_dim * HEAD_BYTES) for _ in range(2)]) for n in (tq, tk, tk)]
+        handle = ctypes.c_void_p()
+        assert ledger.sa_pipeline_create_head_groups(ctypes.byref(handle), 0, *sets, None, 0, 2, tq, tk, 1, 256,
+                                                     q_heads, kv_heads, head_dim, 0, None, None) == 0
+        args = (host.take(tq * row), host.take(tk * row), host.take(tk * row))
+        tail = (cu_q, cu_k, 2, 0.125, 0, 0xC0FFEE, None)
+        if device_output:
+            status = ledger.sa_pipeline_run_device_output(handle, *args, dev.take(tq * row), q_heads * head_dim,
+                                                          head_dim, None, 0, *tail)
+        else:
+            status = ledger.sa_pipeline_run(handle, *args, host.take(tq * row), None, 0, *tail)
+        unfinished = ledger.ledger_unfinished()
+        message = ledger.sa_last_error()
+        assert ledger.sa_pipeline_destroy(handle) == 0
+        return status, unfinished, message
+
+    _fail_each_allocation(ledger, run, f"head groups, device output {device_output}")
+
+
+def test_out_of_host_memory_is_a_return_code_of_resident_and_step_calls(ledger):
+    host = Space(0x5000_0000_0000)
+    cu, b = bounds([300, 200])
+
+    def resident():
+        p = Pipeline(ledger, q_chunk=1024, kv_chunk=256, q_heads=4, kv_heads=2, head_dim=64, num_kv=2, num_out=1)
+        q, out = (p.device_space.take(b[-1] * p.q_row) for _ in range(2))
+        k, v = (p.device_space.take(b[-1] * p.kv_row) for _ in range(2))
+        status = ledger.sa_pipeline_run_resident(p.handle, q, k, v, out, None, 256, 64, 128, 64, 128, 64, 256, 64, 0,
+                                                 cu, cu, 2, 0.125, 0, p.compute, None)
+        message = ledger.sa_last_error()
+        p.destroy()
+        return status, 0, message
+
+    def steps(call):
+        def run():
+            p = Pipeline(ledger, q_chunk=1024, kv_chunk=256, q_heads=4, kv_heads=2, head_dim=64, num_kv=2, num_out=1)
+            assert ledger.sa_pipeline_set_kernel_timing(p.handle, 1) == 0
+            k, v = (host.take(300 * p.kv_row) for _ in range(2))
+            status = call(p, k, v)
+            message = ledger.sa_last_error()
+            assert ledger.sa_pipeline_synchronize(p.handle) == 0
+            p.destroy()
+            return status, 0, message
+        return run
+
+    first = ctypes.c_int32
+    fragments = lambda *addresses: (ctypes.c_void_p * len(addresses))(*addresses)  # noqa: E731
+    rows = (ctypes.c_int32 * 1)(300)
+    tail = lambda p: (900, 0, 0, 0.125, 0, p.compute, None)  # noqa: E731
+    calls = {
+        "stream_kv": lambda p, k, v: ledger.sa_pipeline_stream_kv(p.handle, k, v, 300, *tail(p)),
+        "stream_kv_span": lambda p, k, v: ledger.sa_pipeline_stream_kv_span(
+            p.handle, k, v, 300, 0, ctypes.byref(first(1)), *tail(p)),
+        "stream_kv_gather": lambda p, k, v: ledger.sa_pipeline_stream_kv_gather(
+            p.handle, fragments(k), fragments(v), rows, 1, 0, ctypes.byref(first(1)), *tail(p)),
+    }
+
+    def gather_int8(p, k, v):
+        slots = [(ctypes.c_void_p * 2)(*[p.device_space.take(256 * 2 * 2) for _ in range(2)]) for _ in range(2)]
+        assert ledger.sa_pipeline_attach_int8_scales(p.handle, *slots, 2) == 0
+        scales = [fragments(host.take(300 * 2 * 2)) for _ in range(2)]
+        return ledger.sa_pipeline_stream_kv_gather_int8(p.handle, fragments(k), fragments(v), *scales, rows, 1, 0,
+                                                        ctypes.byref(first(1)), *tail(p))
+
+    _fail_each_allocation(ledger, resident, "resident")
+    for name, call in {**calls, "stream_kv_gather_int8": gather_int8}.items():
+        _fail_each_allocation(ledger, steps(call), name)
