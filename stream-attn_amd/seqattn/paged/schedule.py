@@ -113,7 +113,8 @@ class FragmentQueue:
 
     A fragment that continues the last one within the same allocations joins
     it: one copy of a whole chunk instead of one per page (1 MB pages of 16,384
-    x 16 heads x d128: 128 copies of 24 us with 10-15 us between them).
+    x 16 heads x d128: 128 copies of 24 us with 10-15 us between them).  Rows
+    with an owner to release or with scales of their own stay apart.
     """
 
     row_bytes: int
@@ -127,6 +128,7 @@ class FragmentQueue:
         self.rows += fragment.rows
         last = self.fragments[-1] if self.fragments else None
         if (last is not None and fragment.region is not None and fragment.region == last.region
+                and fragment.owner is None and last.owner is None and not self.scale_row_bytes
                 and fragment.k_address == last.k_address + last.rows * self.row_bytes
                 and fragment.v_address == last.v_address + last.rows * self.row_bytes):
             last.rows += fragment.rows

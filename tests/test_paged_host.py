@@ -282,6 +282,21 @@ def test_fragment_queue_joins_neighbouring_rows_of_one_allocation_only():
     assert done == [None] * 6 and queue.rows == 0
 
 
+def test_fragment_queue_never_joins_rows_that_have_an_owner_or_scales():
+    region = (1000, 5000)
+    queue = FragmentQueue(row_bytes=10)
+    queue.push(Fragment(1000, 5000, 3, "a", region=region))
+    queue.push(Fragment(1030, 5030, 2, "b", region=region))
+    queue.push(Fragment(1050, 5050, 2, region=region))
+    pieces, done = queue.take(7)
+    assert [p[:3] for p in pieces] == [(1000, 5000, 3), (1030, 5030, 2), (1050, 5050, 2)]
+    assert done == ["a", "b", None]
+    queue = FragmentQueue(row_bytes=10, scale_row_bytes=4)
+    queue.push(Fragment(1000, 5000, 3, ks_address=900, vs_address=950, region=region))
+    queue.push(Fragment(1030, 5030, 2, ks_address=800, vs_address=850, region=region))
+    assert queue.take(5)[0] == [(1000, 5000, 3, 900, 950), (1030, 5030, 2, 800, 850)]
+
+
 def test_int8_slots_carry_per_row_scales():
     from seqattn.paged.cache import expand_token_scales, token_scale_layout
     from seqattn.paged.layout import KVLayout, PageDescriptor
