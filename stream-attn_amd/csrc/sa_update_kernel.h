@@ -73,6 +73,134 @@ __device__ inline u32x4 q_sign(float scale_log2) {
   return u32x4{m, m, m, m};
 }
 
+// Fragment reads from LDS.  A batch's reads and the wait for them are one asm
+// statement: the compiler takes an asm's outputs as written when it ends, so a
+// read whose wait stood in a later statement could be copied or overwritten
+// while in flight.  The outputs are early-clobber (later reads of the batch
+// still need the address).  asm rather than plain loads because the compiler
+// cannot relate an LDS read to the DMA writing the other stage and would wait
+// for that prefetch (vmcnt) before it, and because its own schedule waited
+// three times per step (with the second wave of the SIMD usually waiting at
+// the same moment).
+
+// w[kb N / 2 + c] = the 16 bytes at addr + base + kb * step + c KB.
+template <int N>
+__device__ inline __attribute__((always_inline)) void read_k(u32x4 (&w)[N], uint32_t addr, int base, int step) {
+  static_assert(N == 2 || N == 4 || N == 8, "K fragments of a batch");
+  if constexpr (N == 2)
+    asm volatile(
+        "ds_read_b128 %0, %2 offset:%3\n\t"
+        "ds_read_b128 %1, %2 offset:%3+%4\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(w[0]), "=&v"(w[1]) : "v"(addr), "i"(base), "i"(step) : "memory");
+  else if constexpr (N == 4)
+    asm volatile(
+        "ds_read_b128 %0, %4 offset:%5\n\t"
+        "ds_read_b128 %2, %4 offset:%5+%6\n\t"
+        "ds_read_b128 %1, %4 offset:%5+1024\n\t"
+        "ds_read_b128 %3, %4 offset:%5+%6+1024\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3]) : "v"(addr), "i"(base), "i"(step) : "memory");
+  else
+    asm volatile(
+        "ds_read_b128 %0, %8 offset:%9\n\t"
+        "ds_read_b128 %4, %8 offset:%9+%10\n\t"
+        "ds_read_b128 %1, %8 offset:%9+1024\n\t"
+        "ds_read_b128 %5, %8 offset:%9+%10+1024\n\t"
+        "ds_read_b128 %2, %8 offset:%9+2048\n\t"
+        "ds_read_b128 %6, %8 offset:%9+%10+2048\n\t"
+        "ds_read_b128 %3, %8 offset:%9+3072\n\t"
+        "ds_read_b128 %7, %8 offset:%9+%10+3072\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3]), "=&v"(w[4]), "=&v"(w[5]), "=&v"(w[6]), "=&v"(w[7])
+        : "v"(addr), "i"(base), "i"(step)
+        : "memory");
+}
+
+// w[dd] = the 16 bytes at addr + base + dd KB.
+template <int N>
+__device__ inline __attribute__((always_inline)) void read_vt(u32x4 (&w)[N], uint32_t addr, int base) {
+  static_assert(N == 4 || N == 8, "V^T fragments of a batch");
+  if constexpr (N == 4)
+    asm volatile(
+        "ds_read_b128 %0, %4 offset:%5\n\t"
+        "ds_read_b128 %1, %4 offset:%5+1024\n\t"
+        "ds_read_b128 %2, %4 offset:%5+2048\n\t"
+        "ds_read_b128 %3, %4 offset:%5+3072\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3]) : "v"(addr), "i"(base) : "memory");
+  else
+    asm volatile(
+        "ds_read_b128 %0, %8 offset:%9\n\t"
+        "ds_read_b128 %1, %8 offset:%9+1024\n\t"
+        "ds_read_b128 %2, %8 offset:%9+2048\n\t"
+        "ds_read_b128 %3, %8 offset:%9+3072\n\t"
+        "ds_read_b128 %4, %8 offset:%9+4096\n\t"
+        "ds_read_b128 %5, %8 offset:%9+5120\n\t"
+        "ds_read_b128 %6, %8 offset:%9+6144\n\t"
+        "ds_read_b128 %7, %8 offset:%9+7168\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3]), "=&v"(w[4]), "=&v"(w[5]), "=&v"(w[6]), "=&v"(w[7])
+        : "v"(addr), "i"(base)
+        : "memory");
+}
+
+// w[dd]: d block dd of the batch (an even one first) from V's rows, its two
+// 16-key blocks 1 KB apart, each pair of d blocks 4 KB from the next; the odd
+// block of a pair is read at addr_odd.
+template <int N>
+__device__ inline __attribute__((always_inline)) void read_v(u32x4 (&w)[N], uint32_t addr, uint32_t addr_odd, int base) {
+  static_assert(N == 2 || N == 4 || N == 8, "V fragments of a batch");
+  u32x2 h[2 * N];
+  if constexpr (N == 2)
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %4 offset:%6\n\t"
+        "ds_read_b64_tr_b16 %1, %4 offset:%6+1024\n\t"
+        "ds_read_b64_tr_b16 %2, %5 offset:%6\n\t"
+        "ds_read_b64_tr_b16 %3, %5 offset:%6+1024\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(h[0]), "=&v"(h[1]), "=&v"(h[2]), "=&v"(h[3]) : "v"(addr), "v"(addr_odd), "i"(base) : "memory");
+  else if constexpr (N == 4)
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %8 offset:%10\n\t"
+        "ds_read_b64_tr_b16 %1, %8 offset:%10+1024\n\t"
+        "ds_read_b64_tr_b16 %2, %9 offset:%10\n\t"
+        "ds_read_b64_tr_b16 %3, %9 offset:%10+1024\n\t"
+        "ds_read_b64_tr_b16 %4, %8 offset:%10+4096\n\t"
+        "ds_read_b64_tr_b16 %5, %8 offset:%10+5120\n\t"
+        "ds_read_b64_tr_b16 %6, %9 offset:%10+4096\n\t"
+        "ds_read_b64_tr_b16 %7, %9 offset:%10+5120\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(h[0]), "=&v"(h[1]), "=&v"(h[2]), "=&v"(h[3]), "=&v"(h[4]), "=&v"(h[5]), "=&v"(h[6]), "=&v"(h[7])
+        : "v"(addr), "v"(addr_odd), "i"(base)
+        : "memory");
+  else
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %16 offset:%18\n\t"
+        "ds_read_b64_tr_b16 %1, %16 offset:%18+1024\n\t"
+        "ds_read_b64_tr_b16 %2, %17 offset:%18\n\t"
+        "ds_read_b64_tr_b16 %3, %17 offset:%18+1024\n\t"
+        "ds_read_b64_tr_b16 %4, %16 offset:%18+4096\n\t"
+        "ds_read_b64_tr_b16 %5, %16 offset:%18+5120\n\t"
+        "ds_read_b64_tr_b16 %6, %17 offset:%18+4096\n\t"
+        "ds_read_b64_tr_b16 %7, %17 offset:%18+5120\n\t"
+        "ds_read_b64_tr_b16 %8, %16 offset:%18+8192\n\t"
+        "ds_read_b64_tr_b16 %9, %16 offset:%18+9216\n\t"
+        "ds_read_b64_tr_b16 %10, %17 offset:%18+8192\n\t"
+        "ds_read_b64_tr_b16 %11, %17 offset:%18+9216\n\t"
+        "ds_read_b64_tr_b16 %12, %16 offset:%18+12288\n\t"
+        "ds_read_b64_tr_b16 %13, %16 offset:%18+13312\n\t"
+        "ds_read_b64_tr_b16 %14, %17 offset:%18+12288\n\t"
+        "ds_read_b64_tr_b16 %15, %17 offset:%18+13312\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(h[0]), "=&v"(h[1]), "=&v"(h[2]), "=&v"(h[3]), "=&v"(h[4]), "=&v"(h[5]), "=&v"(h[6]), "=&v"(h[7]),
+          "=&v"(h[8]), "=&v"(h[9]), "=&v"(h[10]), "=&v"(h[11]), "=&v"(h[12]), "=&v"(h[13]), "=&v"(h[14]), "=&v"(h[15])
+        : "v"(addr), "v"(addr_odd), "i"(base)
+        : "memory");
+#pragma unroll
+  for (int dd = 0; dd < N; ++dd) w[dd] = u32x4{h[2 * dd][0], h[2 * dd][1], h[2 * dd + 1][0], h[2 * dd + 1][1]};
+}
+
 // DP: head_dim padded to 32, 64, 128 or 256.
 template <int DP>
 struct Geometry {
@@ -390,22 +518,9 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
       const uint32_t k_addr = (uint32_t)(uintptr_t)(const SA_LDS uint8_t*)(k_stage) + k_lane;
 #pragma unroll
       for (int c0 = 0; c0 < CK; c0 += KB) {
-        // The batch's K fragments are read before one wait (the compiler's
-        // own schedule waited three times per step, with the second wave of
-        // the SIMD usually waiting at the same moment).
+        // kf[kb KB + c]: 16-key block kb of the step, d step c0 + c.
         u32x4 kf[2 * KB];
-#pragma unroll
-        for (int c = 0; c < KB; ++c)
-#pragma unroll
-          for (int kb = 0; kb < 2; ++kb) {
-            u32x4 w;
-            asm volatile("ds_read_b128 %0, %1 offset:%2"
-                         : "=v"(w) : "v"(k_addr), "i"(((rb / 16 + kb) * CK + c0 + c) * 1024));
-            kf[kb * KB + c] = w;
-          }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-        for (int x = 0; x < 2 * KB; ++x) asm volatile("" : "+v"(kf[x]));
+        read_k(kf, k_addr, (rb / 16 * CK + c0) * 1024, CK * 1024);
         // Query blocks in snake order: consecutive MFMAs change only one of
         // their A and B operands except where c changes.  An MFMA whose A
         // and B both differ from the previous one's issues later (measured:
@@ -495,43 +610,21 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) l_part[qb] += psum[qb];
 
-      // O^T += V^T P^T, two d blocks per batch of LDS reads.  The reads are
-      // inline asm followed by one explicit lgkmcnt wait: the compiler cannot
-      // relate a transposing LDS read to the DMA writing the other stage and
-      // would otherwise wait for that prefetch (vmcnt) before every read.
-      // LDS reads complete in order, so the compiler's own lgkmcnt waits
-      // around these remain sufficient.
+      // O^T += V^T P^T, VB d blocks per batch of LDS reads.
       const uint32_t v_base = (uint32_t)(uintptr_t)(const SA_LDS uint8_t*)(v_stage);
       const uint32_t v_addr = v_base + v_lane;
       const uint32_t v_addr_odd = v_base + v_lane_odd;
 #pragma unroll
       for (int d0 = 0; d0 < DB; d0 += VB) {
+        // Rows d = 16 db + r16 of V^T, key granule j of the step's 32-key
+        // block.  From V's rows lane (j, r16) addresses key 4 j + r16 / 4 of
+        // each 16-key block at d = 16 db + 4 (r16 % 4) .. +3; after the
+        // transpose it holds d = 16 db + r16 for keys 4 j .. 4 j + 3.
         u32x4 vf[VB];
-#pragma unroll
-        for (int dd = 0; dd < VB; ++dd) {
-          const int db = d0 + dd;
-          if constexpr (VT) {
-            // Rows d = 16 db + r16, key granule j of the step's 32-key block.
-            u32x4 w;
-            asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(w) : "v"(v_addr), "i"(((rb / 32) * DB + db) * 1024));
-            vf[dd] = w;
-          } else {
-            // Lane (j, r16) addresses key 4 j + r16 / 4 of each 16-key block
-            // at d = 16 db + 4 (r16 % 4) .. +3; after the transpose it holds
-            // d = 16 db + r16 for keys 4 j .. 4 j + 3.
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-              u32x2 w;
-              asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2"
-                           : "=v"(w) : "v"(db % 2 ? v_addr_odd : v_addr), "i"((db / 2) * 4096 + (rb + 16 * kb) * 64));
-              vf[dd][2 * kb] = w[0];
-              vf[dd][2 * kb + 1] = w[1];
-            }
-          }
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-        for (int dd = 0; dd < VB; ++dd) asm volatile("" : "+v"(vf[dd]));
+        if constexpr (VT)
+          read_vt(vf, v_addr, (rb / 32 * DB + d0) * 1024);
+        else
+          read_v(vf, v_addr, v_addr_odd, d0 / 2 * 4096 + rb * 64);
 #pragma unroll
         for (int dd = 0; dd < VB; ++dd)
 #pragma unroll
