@@ -5,7 +5,8 @@
  * point takes plain device or pinned-host pointers, element strides and sizes;
  * no C++ type or exception crosses this boundary.  The caller owns all memory:
  * the library never allocates or frees caller buffers.  A pipeline object owns
- * only its own HIP streams and events.
+ * only its own HIP streams and events; pipelines that are given copy streams
+ * share one more stream per device (sa_pipeline_create).
  *
  * Return codes: 0 on success, a positive hipError_t when the HIP runtime
  * failed, or one of the negative SA_ERR_* codes when an argument was rejected.
@@ -182,6 +183,14 @@ typedef struct sa_pipeline_stats {
  *                 destroys with itself.  Caller streams must outlive the
  *                 pipeline; a caller whose allocator tracks stream uses of
  *                 its buffers (torch record_stream) must pass its own streams.
+ *
+ * A pipeline also uses a second launch stream beside compute_stream.  With
+ * NULL copy streams it is the pipeline's own, destroyed with it.  Pipelines on
+ * a device that are given copy streams share one, which the library creates
+ * with the first of them and keeps until the process ends: their launches on
+ * it run in the order they were enqueued, so pipelines that must not wait for
+ * each other's launches pass NULL.  Destroying a pipeline, and an error
+ * return, wait for its own launches there only.
  * All buffers are contiguous.
  */
 int32_t sa_pipeline_create(
@@ -209,7 +218,7 @@ int32_t sa_pipeline_create(
  *                sa_pipeline_attach_resident_scratch (used when a segment's
  *                group_kv_heads * 128 * roundup(keys, 64) * 2 bytes fit)
  *   num_sets     1 or 2; with 2, unit u uses set u % 2 and units alternate
- *                between compute_stream and a second stream of the pipeline,
+ *                between compute_stream and the second launch stream,
  *                and the units' sizes ramp up 1, 2, 4, ... K/V heads and back
  *                down at the end, with units of at most group_kv_heads,
  *                evened out, between (the first unit's copies and the last
@@ -273,9 +282,9 @@ int32_t sa_pipeline_destroy(sa_pipeline* pipeline);
  * block's first chunk is copied ahead of its Q rows and applied to each
  * piece as its rows land; every row still sees the same chunks in the same
  * order.  Returns after the D2H stream has drained.  An error return comes
- * after the pipeline's copy streams and second stream have drained, so no
- * copy still reads or writes the host buffers; launches already enqueued on
- * compute_stream may still run.
+ * after the pipeline's copy streams have drained and its launches on the
+ * second stream have ended, so no copy still reads or writes the host buffers;
+ * launches already enqueued on compute_stream may still run.
  *
  *   q_host/k_host/v_host/out_host: contiguous pinned host [tokens, heads, head_dim] dtype
  *   cu_seqlens_q/k: num_segments + 1 host int64 boundaries
@@ -298,8 +307,7 @@ int32_t sa_pipeline_run(
  * output copy is made.  Enqueued on compute_stream (and the pipeline's
  * second stream, joined back into it); returns once the host inputs have
  * been copied, before the launches end: later work on compute_stream sees
- * the output and the LSE.  An error return comes after the copy streams and
- * the second stream have drained, as for sa_pipeline_run.  No counterpart in
+ * the output and the LSE.  An error return waits as sa_pipeline_run's does.  No counterpart in
  * the reference (its device outputs go through output_transform,
  * executor.py:145-172).
  */

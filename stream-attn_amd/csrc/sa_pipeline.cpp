@@ -20,9 +20,11 @@
 // finalize of this file read and write; the buffers must therefore hold the
 // Q block's rows rounded up to a multiple of 16.
 //
-// Streamed chunks of a Q block of at least 512 rows are applied by two
-// launches, one per half of the block's rows: the first on the compute
-// stream, the second on the pipelines' `side` stream (default priority).
+// Streamed chunks of a Q block of at least two workgroup tiles (twice
+// update_block_rows: 512 rows up to head_dim 64, 768 up to 128, 256 above) are
+// applied by two launches, one per half of the block's rows: the first on the
+// compute stream, the second on the `side` stream (default priority; see
+// acquire_side).
 // A span forks `side` from the compute stream and joins it back, and a slot
 // is refilled only after both halves recorded their kv_free events.  The two
 // halves' launches run concurrently, so one launch's partial last round of
@@ -146,6 +148,7 @@ struct sa_pipeline {
   // Second half of a split chunk update: its stream, the slot-free events it
   // records, and the span's fork / join events.
   hipStream_t side = nullptr;
+  bool owns_side = false;
   hipEvent_t kv_free_side[3] = {};
   hipEvent_t fork = nullptr, join = nullptr;
   bool kv_side_pending[3] = {false, false, false};
@@ -205,51 +208,51 @@ void add_stats(sa_pipeline_stats* st, int64_t h2d, int64_t d2h, int64_t qc, int6
   st->max_resident_q_tokens = std::max(st->max_resident_q_tokens, resident);
 }
 
-// The second launch stream of every pipeline on a device: created with the
-// first of them, destroyed with the last.  HIP deals streams onto a few
-// hardware queues as they are created; with a stream per pipeline the third
-// runner's landed on a queue of the other streams, and its two launch streams
-// took turns (65,536 x 32 heads in head groups: 75 ms a run instead of 58).
-// Launches of different pipelines on it run in order, like their copies on
-// the shared copy streams; everything a launch waits for was enqueued before
-// it, so none can wait for another's later work.
-struct SideStream {
-  hipStream_t stream = nullptr;
-  int users = 0;
-};
+// The second launch stream.  Pipelines that are given their copy streams share
+// one per device, created with the first of them and kept until the process
+// ends, like the streams they are given; a pipeline that makes its own copy
+// streams makes its own second stream too.  HIP deals streams onto a few
+// hardware queues in the order they are created, so a stream made with each
+// pipeline lands on a queue that depends on what was made before it: with
+// three runners alive the third one's was the queue of another stream it
+// uses, and its two launch streams took turns (65,536 x 32 heads in head
+// groups, one box: the first runner 65 ms a run and the third 81 with a stream
+// each, every runner 61 with the shared one, also after others were closed).
+// Launches of different pipelines on the shared stream run in order, like
+// their copies; everything a launch waits for was enqueued before it, so none
+// can wait for another's later work.
 constexpr int kSideDevices = 64;  // pipelines on a device past these have a stream each
 std::mutex g_side_mutex;
-SideStream g_side_streams[kSideDevices];
+hipStream_t g_side_streams[kSideDevices];
 
-// The device is current.
+// The device is current and the copy streams are known.
 hipError_t acquire_side(sa_pipeline* p) {
-  if (p->device < 0 || p->device >= kSideDevices) return hipStreamCreateWithFlags(&p->side, hipStreamNonBlocking);
+  p->owns_side = p->owns_streams || p->device < 0 || p->device >= kSideDevices;
+  if (p->owns_side) return hipStreamCreateWithFlags(&p->side, hipStreamNonBlocking);
   std::lock_guard<std::mutex> lock(g_side_mutex);
-  SideStream& side = g_side_streams[p->device];
-  if (side.users == 0) {
-    const hipError_t err = hipStreamCreateWithFlags(&side.stream, hipStreamNonBlocking);
+  hipStream_t& shared = g_side_streams[p->device];
+  if (!shared) {
+    hipStream_t made = nullptr;
+    const hipError_t err = hipStreamCreateWithFlags(&made, hipStreamNonBlocking);
     if (err != hipSuccess) return err;
+    shared = made;
   }
-  ++side.users;
-  p->side = side.stream;
+  p->side = shared;
   return hipSuccess;
 }
 
-void release_side(sa_pipeline* p) {
-  const hipStream_t stream = std::exchange(p->side, nullptr);
-  if (p->device < 0 || p->device >= kSideDevices) {
-    (void)hipStreamDestroy(stream);
-    return;
-  }
-  std::lock_guard<std::mutex> lock(g_side_mutex);
-  if (--g_side_streams[p->device].users == 0) (void)hipStreamDestroy(stream);
+// Waits for this pipeline's launches on the second stream, which every span
+// and run ends with the `join` event (SideJoin); not for what others have
+// enqueued on a shared stream meanwhile.
+void wait_side(sa_pipeline* p) {
+  if (p->join) (void)hipEventSynchronize(p->join);
 }
 
 // Teardown: failures here cannot be acted on, so their codes are dropped.
 void release(sa_pipeline* p) {
   if (p->h2d) (void)hipStreamSynchronize(p->h2d);
   if (p->d2h) (void)hipStreamSynchronize(p->d2h);
-  if (p->side) (void)hipStreamSynchronize(p->side);
+  wait_side(p);
   hipEvent_t* evs[] = {&p->q_ready, &p->q_free, &p->fork, &p->join};
   for (hipEvent_t* e : evs)
     if (*e) (void)hipEventDestroy(*e);
@@ -283,7 +286,7 @@ void release(sa_pipeline* p) {
     if (p->h2d) (void)hipStreamDestroy(p->h2d);
     if (p->d2h) (void)hipStreamDestroy(p->d2h);
   }
-  if (p->side) release_side(p);
+  if (p->side && p->owns_side) (void)hipStreamDestroy(p->side);
 }
 
 // Make the H2D stream wait until ring slot `slot` is no longer read by any
@@ -1079,8 +1082,8 @@ std::vector<int> head_group_unit_sizes(int kv_heads, int group_kv, int num_sets)
 
 // sa_pipeline_run on a head-group pipeline.  Unit u (a range of K/V heads,
 // at most group_kv, with their query heads) uses buffer set u % num_sets
-// and, with two sets, compute stream u % 2 (the caller's, then the
-// pipeline's second stream):
+// and, with two sets, compute stream u % 2 (the caller's, then the second
+// stream):
 //   H2D : [wait set_done] K and V columns of every token, [wait set_free] Q
 //         columns (strided copies from the host's [token][head][d] rows),
 //         record set_ready;
@@ -1370,7 +1373,7 @@ int32_t run_host_output(sa_pipeline* p, const void* q_host, const void* k_host, 
 void drain_after_error(sa_pipeline* p) {
   if (p->h2d) (void)hipStreamSynchronize(p->h2d);
   if (p->d2h) (void)hipStreamSynchronize(p->d2h);
-  if (p->side) (void)hipStreamSynchronize(p->side);
+  wait_side(p);
 }
 
 }  // namespace

@@ -41,8 +41,9 @@ def close_all_workspaces() -> None:
 
     Registered with ``atexit``: it runs before the interpreter tears down
     modules and before the shared libraries' static destructors, so no
-    pipeline (its events and side stream) and no scratch buffer is released
-    after the HIP runtime has begun to shut down.
+    pipeline (its events) and no scratch buffer is released after the HIP
+    runtime has begun to shut down.  The launch stream that the pipelines of a
+    device share is the library's and lives as long as the process.
     """
     for workspace in list(_LIVE):
         try:

@@ -66,6 +66,7 @@ struct Ledger {
   long dropped = 0;
   long copies_seen = 0;
   long fail_copy = -1;
+  long streams_created = 0, streams_destroyed = 0;
 };
 
 Ledger g;
@@ -182,9 +183,13 @@ hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* stream, unsigned int) {
   Recording own;
   *stream = new_handle<hipStream_t>();
+  ++g.streams_created;
   return hipSuccess;
 }
-hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) {
+  ++g.streams_destroyed;
+  return hipSuccess;
+}
 hipError_t hipStreamSynchronize(hipStream_t stream) {
   Recording own;
   push(Op{kStreamSync, stream_id(stream), -1, {}, {}, "stream sync"});
@@ -346,6 +351,7 @@ void ledger_reset(void) {
   g.dropped = 0;
   g.copies_seen = 0;
   g.fail_copy = -1;
+  g.streams_created = g.streams_destroyed = 0;
   g_fail_allocation = -1;
 }
 
@@ -365,6 +371,22 @@ long ledger_copies(void) { return g.copies_seen; }
 long ledger_waits(void) { return g.waits_seen; }
 
 long ledger_dropped(void) { return g.dropped; }
+
+// Streams created and destroyed since the reset.
+void ledger_streams(int64_t* out) {
+  out[0] = g.streams_created;
+  out[1] = g.streams_destroyed;
+}
+
+// Kinds (the order of enum Kind) and streams of up to n recorded operations;
+// returns how many there are.
+int64_t ledger_ops(int32_t* kinds, int32_t* streams, int64_t n) {
+  for (int64_t i = 0; i < n && i < (int64_t)g.ops.size(); ++i) {
+    kinds[i] = g.ops[i].kind;
+    streams[i] = g.ops[i].stream;
+  }
+  return (int64_t)g.ops.size();
+}
 
 // Counts of recorded operations: [copies H2D, copies D2H, kernels, waits].
 void ledger_counts(int64_t* out) {

@@ -58,6 +58,9 @@ def ledger(tmp_path_factory):
     lib.ledger_copies.restype = ctypes.c_long
     lib.ledger_fail_allocation.argtypes = [ctypes.c_long]
     lib.ledger_allocations.restype = ctypes.c_long
+    lib.ledger_streams.argtypes = [ctypes.POINTER(ctypes.c_int64)]
+    lib.ledger_ops.restype = ctypes.c_int64
+    lib.ledger_ops.argtypes = [ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32), ctypes.c_int64]
     lib.ledger_unfinished.restype = ctypes.c_int64
     return lib
 
@@ -75,7 +78,8 @@ class Space:
 
 
 class Pipeline:
-    def __init__(self, lib, *, q_chunk, kv_chunk, q_heads, kv_heads, head_dim, num_kv, num_out, out_slots=True):
+    def __init__(self, lib, *, q_chunk, kv_chunk, q_heads, kv_heads, head_dim, num_kv, num_out, out_slots=True,
+                 copy_streams=(None, None)):
         dev = Space(0x7000_0000_0000)
         q_row = q_heads * head_dim * HEAD_BYTES
         kv_row = kv_heads * head_dim * HEAD_BYTES
@@ -96,7 +100,7 @@ class Pipeline:
         outs = (ctypes.c_void_p * 2)(*self.out_slots) if out_slots else None
         status = lib.sa_pipeline_create(ctypes.byref(handle), 0, self.q_buffer, ks, vs, num_kv, self.m, self.l,
                                          self.acc, outs, num_out, q_chunk, kv_chunk, q_heads, kv_heads, head_dim, 0,
-                                         None, None)
+                                         *copy_streams)
         assert status == 0, lib.sa_last_error()
         self.handle = handle
         self.compute = 0xC0FFEE  # the caller's compute stream handle
@@ -707,3 +711,84 @@ def test_out_of_host_memory_is_a_return_code_of_resident_and_step_calls(ledger):
     _fail_each_allocation(ledger, resident, "resident")
     for name, call in {**calls, "stream_kv_gather_int8": gather_int8}.items():
         _fail_each_allocation(ledger, steps(call), name)
+
+
+KERNEL, STREAM_SYNC, EVENT_SYNC = 3, 6, 7  # enum Kind of fence_ledger.cpp
+
+
+def _operations(ledger):
+    n = ledger.ledger_ops(None, None, 0)
+    kinds, streams = (ctypes.c_int32 * n)(), (ctypes.c_int32 * n)()
+    ledger.ledger_ops(kinds, streams, n)
+    return list(zip(kinds, streams))
+
+
+def _split_run(ledger, p, host):
+    """A run whose Q block is wide enough for two launches a chunk."""
+    cu, b = bounds([1500])
+    out = host.take(b[-1] * p.q_row)
+    assert ledger.sa_pipeline_run(p.handle, host.take(b[-1] * p.q_row), host.take(b[-1] * p.kv_row),
+                                  host.take(b[-1] * p.kv_row), out, None, 0, cu, cu, 1, 0.125, 0, p.compute, None) == 0
+
+
+def _pipeline(ledger, **kw):
+    return Pipeline(ledger, q_chunk=2048, kv_chunk=512, q_heads=4, kv_heads=2, head_dim=64, num_kv=2, num_out=1, **kw)
+
+
+def test_the_shared_launch_stream_outlives_the_pipelines(ledger):
+    # Pipelines on shared copy streams share their second launch stream; it
+    # is not made anew when the last of them goes (a stream's hardware queue
+    # depends on the order in which streams are created).
+    host = Space(0x5000_0000_0000)
+    p = _pipeline(ledger, copy_streams=(0xA100, 0xA200))  # the shared stream exists from here on
+    p.destroy()
+    ledger.ledger_reset()
+    launches = set()
+    for _ in range(3):
+        p = _pipeline(ledger, copy_streams=(0xA100, 0xA200))
+        _split_run(ledger, p, host)
+        p.destroy()
+        launches |= {stream for kind, stream in _operations(ledger) if kind == KERNEL}
+    counts = (ctypes.c_int64 * 2)()
+    ledger.ledger_streams(counts)
+    assert list(counts) == [0, 0]
+    assert len(launches) == 2  # the compute stream and the shared one
+    check(ledger, "shared launch stream")
+
+
+def test_a_pipeline_with_copy_streams_of_its_own_has_its_own_launch_stream(ledger):
+    host = Space(0x5000_0000_0000)
+    ledger.ledger_reset()
+    pipelines = [_pipeline(ledger) for _ in range(2)]
+    for p in pipelines:
+        _split_run(ledger, p, host)
+    assert len({stream for kind, stream in _operations(ledger) if kind == KERNEL}) == 3
+    for p in pipelines:
+        p.destroy()
+    counts = (ctypes.c_int64 * 2)()
+    ledger.ledger_streams(counts)
+    assert list(counts) == [6, 6]
+    check(ledger, "own launch streams")
+
+
+def test_a_pipeline_waits_for_its_own_work_on_the_shared_launch_stream_only(ledger):
+    # Destroying a pipeline, and a failed run, must not wait for what other
+    # pipelines have enqueued on the shared stream: they follow the event
+    # recorded after their own launches.
+    host = Space(0x5000_0000_0000)
+    ledger.ledger_reset()
+    p = _pipeline(ledger, copy_streams=(0xA100, 0xA200))
+    _split_run(ledger, p, host)
+    shared = {stream for kind, stream in _operations(ledger) if kind == KERNEL}
+    done = len(_operations(ledger))
+    ledger.ledger_fail_copy(ledger.ledger_copies() + 4)
+    cu, b = bounds([1500])
+    assert ledger.sa_pipeline_run(p.handle, host.take(b[-1] * p.q_row), host.take(b[-1] * p.kv_row),
+                                  host.take(b[-1] * p.kv_row), host.take(b[-1] * p.q_row), None, 0, cu, cu, 1, 0.125,
+                                  0, p.compute, None) != 0
+    failed = _operations(ledger)[done:]
+    p.destroy()
+    destroyed = _operations(ledger)[done + len(failed):]
+    for operations in (failed, destroyed):
+        assert not [stream for kind, stream in operations if kind == STREAM_SYNC and stream in shared]
+        assert any(kind == EVENT_SYNC for kind, _ in operations)
