@@ -441,15 +441,25 @@ int32_t sa_pipeline_run_resident(sa_pipeline* pipeline, const void* q, const voi
  * Attach caller-owned device scratch for sa_pipeline_run_resident (NULL and 0
  * detach it).  No counterpart in the reference.  With head_dim 128, a fused
  * resident launch whose segment has kv_tokens keys and at least 65,536
- * queries x query heads per K/V head first copies V into it, transposed per
- * K/V head (128 x the keys padded to a multiple of 64, 16-bit), when
- * kv_heads * 128 * roundup(kv_tokens, 64) * 2 bytes fit; the update kernel
- * then reads V^T fragments with half the LDS instructions.
+ * queries x query heads per K/V head, or whose V has a token stride outside
+ * [1, 2^24) elements (which only the copy can read), first copies V into it,
+ * transposed per K/V head (128 x the keys padded to a multiple of 64, 16-bit),
+ * when kv_heads * 128 * roundup(kv_tokens, 64) * 2 bytes fit; the update
+ * kernel then reads V^T fragments with half the LDS instructions.
  * Results are identical with or without it.  The pipeline keeps the pointer
  * until it is replaced or the pipeline is destroyed; runs on one pipeline
  * share it, in stream order.
  */
 int32_t sa_pipeline_attach_resident_scratch(sa_pipeline* pipeline, void* scratch, int64_t bytes);
+
+/*
+ * The scratch bytes that sa_pipeline_run_resident would use for these segments,
+ * V's token stride and this output (strides as there): the largest of the
+ * copies it makes, 0 when it reads V in place.  Host arithmetic only.
+ */
+int32_t sa_pipeline_resident_scratch_bytes(
+    sa_pipeline* pipeline, int64_t stride_vt, const void* out, int64_t stride_ot, int64_t stride_oh,
+    const int64_t* cu_seqlens_q, const int64_t* cu_seqlens_k, int32_t num_segments, int64_t* bytes);
 
 /*
  * Finalize the resident state on compute_stream (executor.py:125-142).

@@ -1012,6 +1012,31 @@ int32_t fused_merge_keys(const sa_pipeline* p, int64_t k_length) {
   return k_length <= p->kv_chunk ? 0 : -1;
 }
 
+// How sa_pipeline_run_resident takes a segment: as one fused launch (alone or
+// with others) that merges its row sums every `merge` keys, or (not fused)
+// through the chunked schedule; and the bytes of the transposed copy of V made
+// before that launch (0: V is read in place).
+struct ResidentSegment {
+  bool fused;
+  int32_t merge;
+  int64_t vt_bytes;
+};
+
+ResidentSegment resident_segment(const sa_pipeline* p, int64_t q_length, int64_t k_length, int64_t stride_vt,
+                                 const char* seg_out, int64_t stride_ot, int64_t stride_oh) {
+  ResidentSegment r{};
+  // A head-group pipeline has no Q block or state buffers: only the single
+  // fused launch is available to it.
+  r.merge = p->head_groups ? fused_merge_keys(p, k_length) : (p->kv_chunk % 64 == 0 ? p->kv_chunk : -1);
+  r.fused = q_length > 0 && r.merge >= 0 && q_length <= INT32_MAX && k_length <= INT32_MAX && stride_ot % 8 == 0 &&
+            stride_oh % 8 == 0 && reinterpret_cast<uintptr_t>(seg_out) % 16 == 0;
+  const int64_t t_pad = (k_length + 63) / 64 * 64;
+  if (r.fused && p->head_dim == 128 && t_pad < (1 << 24) &&
+      sa::transposes_v(q_length, p->q_heads / p->kv_heads, stride_vt))
+    r.vt_bytes = (int64_t)p->kv_heads * 128 * t_pad * 2;
+  return r;
+}
+
 // One fused update launch of the head-group schedule (initializes, runs over
 // every key of a segment, writes the output and the LSE), optionally
 // bracketed by timing events.
@@ -1806,19 +1831,14 @@ int32_t sa_pipeline_run_resident(sa_pipeline* p, const void* q, const void* k, c
     KVSource src{kd + k_start * stride_kt * 2, vd + k_start * stride_vt * 2, true,
                  stride_kt, stride_kh, stride_vt, stride_vh};
     char* seg_out = od + q_start * stride_ot * 2;
-    // A head-group pipeline has no Q block or state buffers: only the single
-    // fused launch below is available to it.
-    const int32_t merge = p->head_groups ? fused_merge_keys(p, k_length) : (p->kv_chunk % 64 == 0 ? p->kv_chunk : -1);
-    const bool fused_segment = q_length > 0 && merge >= 0 && q_length <= INT32_MAX && k_length <= INT32_MAX &&
-                               stride_ot % 8 == 0 && stride_oh % 8 == 0 &&
-                               reinterpret_cast<uintptr_t>(seg_out) % 16 == 0;
-    if (p->head_groups && q_length > 0 && !fused_segment) {
+    const ResidentSegment how = resident_segment(p, q_length, k_length, stride_vt, seg_out, stride_ot, stride_oh);
+    if (p->head_groups && q_length > 0 && !how.fused) {
       sa::set_error("sa_pipeline_run_resident: segment %d needs the chunked schedule (a 16-byte aligned output "
                     "with strides that are multiples of 8, and at most one K/V chunk unless the chunk is a "
                     "multiple of 64), which a head-group pipeline does not have", s);
       return SA_ERR_BAD_STATE;
     }
-    if (fused_segment) {
+    if (how.fused) {
       // K/V already in HBM: one launch covers every query and key of the
       // segment and finalizes its rows in the epilogue.  The row sums are
       // merged at every kv_chunk boundary exactly as the chunked schedule
@@ -1832,9 +1852,7 @@ int32_t sa_pipeline_run_resident(sa_pipeline* p, const void* q, const void* k, c
       // for the same operands; the other segments go together in one launch
       // after the loop.
       const int64_t t_pad = (k_length + 63) / 64 * 64;
-      const int64_t vt_bytes = (int64_t)p->kv_heads * 128 * t_pad * 2;
-      const bool vt = p->head_dim == 128 && p->vt_scratch != nullptr && vt_bytes <= p->vt_scratch_bytes &&
-                      t_pad < (1 << 24) && sa::transposes_v(q_length, p->q_heads / p->kv_heads, stride_vt);
+      const bool vt = how.vt_bytes > 0 && p->vt_scratch != nullptr && how.vt_bytes <= p->vt_scratch_bytes;
       if (vt || !together.add(q_start, q_length, k_start, k_length)) {
         int32_t rc = 0;
         if (vt) {
@@ -1846,11 +1864,11 @@ int32_t sa_pipeline_run_resident(sa_pipeline* p, const void* q, const void* k, c
         rc = launch_timed(p, qd + q_start * stride_qt * 2, stride_qt, stride_qh, src.k, src.sk_t, src.sk_h,
                           vt ? static_cast<const char*>(p->vt_scratch) : src.v, vt ? t_pad : src.sv_t,
                           vt ? 128 * t_pad : src.sv_h, (int32_t)q_length, (int32_t)k_length, 0, 0, causal_shift,
-                          softmax_scale, (causal ? SA_FLAG_CAUSAL : 0) | SA_FLAG_INITIALIZE, compute, merge,
-                          &fused, 0, vt);
+                          softmax_scale, (causal ? SA_FLAG_CAUSAL : 0) | SA_FLAG_INITIALIZE, compute,
+                          how.merge, &fused, 0, vt);
         if (rc != 0) return rc;
       } else {
-        together_merge = merge;
+        together_merge = how.merge;
       }
       const int64_t block = p->head_groups ? q_length
                                            : pass_rows(q_length, p->q_chunk, sa::update_block_rows(p->head_dim));
@@ -1898,6 +1916,25 @@ int32_t sa_pipeline_run_resident(sa_pipeline* p, const void* q, const void* k, c
   return 0;
 } catch (const std::exception& error) {
   return sa::exception_status("sa_pipeline_run_resident", error);
+}
+
+int32_t sa_pipeline_resident_scratch_bytes(sa_pipeline* p, int64_t stride_vt, const void* out, int64_t stride_ot,
+                                           int64_t stride_oh, const int64_t* cu_seqlens_q,
+                                           const int64_t* cu_seqlens_k, int32_t num_segments, int64_t* bytes) {
+  sa::clear_error();
+  if (!p || !cu_seqlens_q || !cu_seqlens_k || num_segments < 0 || !bytes) {
+    sa::set_error("sa_pipeline_resident_scratch_bytes: null argument");
+    return SA_ERR_INVALID_ARGUMENT;
+  }
+  *bytes = 0;
+  for (int32_t s = 0; s < num_segments; ++s) {
+    const char* seg_out = static_cast<const char*>(out) + cu_seqlens_q[s] * stride_ot * 2;
+    const ResidentSegment how =
+        resident_segment(p, cu_seqlens_q[s + 1] - cu_seqlens_q[s], cu_seqlens_k[s + 1] - cu_seqlens_k[s], stride_vt,
+                         seg_out, stride_ot, stride_oh);
+    *bytes = std::max(*bytes, how.vt_bytes);
+  }
+  return 0;
 }
 
 int32_t sa_pipeline_finalize(sa_pipeline* p, int32_t slot, int32_t q_tokens, float* lse,

@@ -146,10 +146,17 @@ class HipExecutorMixin:
         self._check_lse(lse, q.shape[0])
         native_stats = _native.PipelineStats()
         compute = workspace.compute_stream
-        longest_k = max((b - a for a, b in zip(k_bounds[:-1], k_bounds[1:])), default=0)
-        stats.resident_scratch_bytes = workspace.attach_resident_scratch(
-            longest_k, self.config.resident_scratch_limit_bytes
-        )
+        bounds = (_bounds_array(q_bounds), _bounds_array(k_bounds), len(q_bounds) - 1)
+        stats.resident_scratch_bytes = 0
+        if self.plan.head_dim == 128:
+            needed = ctypes.c_int64()
+            status = _native.lib().sa_pipeline_resident_scratch_bytes(
+                workspace.handle, v.stride(0), out.data_ptr(), *out.stride()[:2], *bounds, ctypes.byref(needed)
+            )
+            _native.check(status, "sa_pipeline_resident_scratch_bytes")
+            stats.resident_scratch_bytes = workspace.attach_resident_scratch(
+                needed.value, self.config.resident_scratch_limit_bytes
+            )
         # The usual caller is on the compute stream itself, and the native
         # call selects the device by itself: no device or stream object is
         # made then (about a third of a short call's host time).
@@ -165,8 +172,7 @@ class HipExecutorMixin:
                 None if lse is None else lse.data_ptr(),
                 *q.stride()[:2], *k.stride()[:2], *v.stride()[:2], *out.stride()[:2],
                 0 if lse is None else lse.stride(0),
-                _bounds_array(q_bounds), _bounds_array(k_bounds), len(q_bounds) - 1,
-                float(scale), int(bool(causal)),
+                *bounds, float(scale), int(bool(causal)),
                 compute_ptr, ctypes.byref(native_stats),
             )
         _native.check(status, "sa_pipeline_run_resident")

@@ -181,23 +181,22 @@ class CudaWorkspace:
         )
         _native.check(status, "sa_pipeline_attach_resident_scratch")
 
-    def attach_resident_scratch(self, kv_tokens: int, limit_bytes: int | None = None) -> int:
+    def attach_resident_scratch(self, needed: int, limit_bytes: int | None = None) -> int:
         """HBM-resident runs with head_dim 128: device scratch for V
         transposed per K/V head, [kv_heads, 128, kv_tokens padded to a
         multiple of 64] 16-bit elements, which the update kernel reads with
-        half the LDS instructions (in segments of enough queries to repay the
-        copy).  Grown on demand and kept for later runs; outside the planner's
-        workspace budget, like the resident inputs.
+        half the LDS instructions.  ``needed`` is the largest copy that the
+        run makes (sa_pipeline_resident_scratch_bytes: segments of enough
+        queries to repay it), 0 for most.  Grown on demand and kept for later
+        runs; outside the planner's workspace budget, like the resident inputs.
 
-        Returns the scratch bytes the next run may use, 0 when it reads V in
+        Returns the scratch bytes the next run will use, 0 when it reads V in
         place instead: ``limit_bytes`` caps the scratch (0 disables it), and
         an allocation that fails for lack of device memory also leaves the
         run on the in-place path, which gives the same results bit for bit.
         """
-        plan = self.plan
-        if plan.head_dim != 128 or kv_tokens <= 0:
+        if needed <= 0:
             return 0
-        needed = plan.kv_heads * 128 * ((kv_tokens + 63) // 64 * 64) * 2
         if self.resident_scratch is not None and self.resident_scratch.numel() >= needed:
             return needed
         if limit_bytes is not None and needed > limit_bytes:

@@ -792,3 +792,53 @@ def test_a_pipeline_waits_for_its_own_work_on_the_shared_launch_stream_only(ledg
     for operations in (failed, destroyed):
         assert not [stream for kind, stream in operations if kind == STREAM_SYNC and stream in shared]
         assert any(kind == EVENT_SYNC for kind, _ in operations)
+
+
+@pytest.mark.parametrize("q_lengths,k_lengths,heads,head_dim,kv_chunk,stride_vt,copies,longest", [
+    # Few queries: a decoding step and the continuation of a long context.
+    ([1, 1], [8000, 400], (8, 2), 128, 256, 256, 0, 0),
+    ([1009], [61312], (32, 8), 128, 256, 1024, 0, 0),
+    # 65,536 queries x heads per K/V head and more; the longest segment does
+    # not take part.
+    ([2048, 2047, 2100], [999, 5000, 1300], (32, 1), 128, 256, 128, 2, 1300),
+    # V token strides that only the copy can read.
+    ([5, 0, 70], [3, 900, 64], (4, 2), 128, 256, 0, 2, 64),
+    ([5], [3], (4, 2), 128, 256, 1 << 24, 1, 3),
+    # Another head_dim, and a chunk that keeps the run out of the fused launch.
+    ([70000], [100], (4, 4), 64, 256, 256, 0, 0),
+    ([70000], [100], (4, 4), 128, 100, 512, 0, 0),
+])
+def test_resident_scratch_is_what_the_run_reads(ledger, q_lengths, k_lengths, heads, head_dim, kv_chunk, stride_vt,
+                                                copies, longest):
+    q_heads, kv_heads = heads
+    cu_q, q_b = bounds(q_lengths)
+    cu_k, k_b = bounds(k_lengths)
+    p = Pipeline(ledger, q_chunk=1024, kv_chunk=kv_chunk, q_heads=q_heads, kv_heads=kv_heads, head_dim=head_dim,
+                 num_kv=2, num_out=1)
+    dev = p.device_space
+    q, out = dev.take(q_b[-1] * p.q_row), dev.take(q_b[-1] * p.q_row)
+    k, v = dev.take(k_b[-1] * p.kv_row), dev.take(k_b[-1] * max(stride_vt, 1) * HEAD_BYTES)
+    qs, ks = (q_heads * head_dim, head_dim), (kv_heads * head_dim, head_dim)
+    needed = ctypes.c_int64(-1)
+    assert ledger.sa_pipeline_resident_scratch_bytes(p.handle, stride_vt, out, *qs, cu_q, cu_k, len(q_lengths),
+                                                     ctypes.byref(needed)) == 0
+    assert needed.value == kv_heads * 128 * (-(-longest // 64) * 64) * HEAD_BYTES
+
+    def launches(scratch_bytes):
+        ledger.ledger_reset()
+        assert ledger.sa_pipeline_attach_resident_scratch(p.handle, dev.take(scratch_bytes) if scratch_bytes else None,
+                                                          scratch_bytes) == 0
+        assert ledger.sa_pipeline_run_resident(p.handle, q, k, v, out, None, *qs, *ks, stride_vt, head_dim, *qs, 0, cu_q,
+                                               cu_k, len(q_lengths), 0.1, 0, p.compute, None) == 0
+        counts = (ctypes.c_int64 * 4)()
+        ledger.ledger_counts(counts)
+        return counts[2]
+
+    # Each copy is one launch, and its segment then has an update launch of
+    # its own; the others go together.
+    others = sum(1 for n in q_lengths if n) - copies
+    if kv_chunk % 64 == 0:
+        assert launches(needed.value) == 2 * copies + (others > 0)
+        assert launches(0) == 1
+    assert launches(needed.value) == launches(1 << 40)  # more scratch changes nothing
+    p.destroy()
