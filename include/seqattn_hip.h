@@ -86,6 +86,20 @@ int32_t sa_update_attention_state(
     void* stream);
 
 /*
+ * The shape of the update launch over up to 32 segments of (q_tokens[i] > 0,
+ * kv_tokens[i]): the query rows of a workgroup, its LDS stages and the number
+ * of workgroups.  A diagnostic: results do not depend on it.  Host arithmetic
+ * only.  With one segment query i sees the keys up to i + causal_shift; several
+ * are each bottom-right causal.  kv_layout: 0 for 16-bit K and V, 1 for the
+ * transposed copy of V (head_dim 128), 2 for INT8 (1 and 2: one segment);
+ * overlapped: another launch of about this size runs beside it.
+ */
+int32_t sa_update_launch_shape(
+    const int32_t* q_tokens, const int32_t* kv_tokens, int32_t num_segments, int32_t q_heads, int32_t kv_heads,
+    int32_t head_dim, int32_t causal_shift, int32_t causal, int32_t kv_layout, int32_t overlapped, int32_t* rows,
+    int32_t* stages, int64_t* workgroups);
+
+/*
  * The update above with INT8 K/V and per-group fp16 scales.
  *
  * Replaces update_attention_state_int8 (reference

@@ -206,15 +206,74 @@ int choose_rows(const UpdateParams& p, int d, int mode, bool overlapped) {
   return rows;
 }
 
+// Numbers the launch's workgroups of `rows` rows (p's pack, unit_heads,
+// numbering, first, slots and xcd_run) and returns how many there are.
+uint32_t number_workgroups(UpdateParams& p, int rows) {
+  const bool several = p.segments > 1;
+  int64_t most_queries = several ? 0 : p.q_tokens;
+  for (int s = 0; several && s < p.segments; ++s) most_queries = std::max<int64_t>(most_queries, p.segment[s].q_len);
+  p.pack = rows == kRowsPerBlock && p.group > 1 && most_queries * p.group <= INT32_MAX;
+  p.unit_heads = p.pack ? p.q_heads / p.group : p.q_heads;
+  p.numbering = p.unit_heads % 8 == 0 ? kHeadsPerXcd : p.causal || several ? kDealt : kRunsPerXcd;
+  const int heads = p.numbering == kHeadsPerXcd ? p.unit_heads / 8 : p.unit_heads;
+  const int per_query = p.pack ? p.group : 1;
+  p.slots = 0;
+  for (int s = 0; s < (several ? p.segments : 1); ++s) {
+    p.first[s] = p.slots;
+    const int64_t queries = several ? p.segment[s].q_len : p.q_tokens;
+    p.slots += (int32_t)((queries * per_query + rows - 1) / rows * heads);
+  }
+  p.xcd_run = (p.slots + 7) / 8;
+  return p.numbering == kHeadsPerXcd ? 8u * p.slots : p.numbering == kDealt ? p.slots : 8u * p.xcd_run;
+}
+
+// LDS stages of a launch.  With two, a workgroup alone on its CU waits at
+// every barrier for the tile it just requested; with four it has three tiles
+// in flight, but starts later and runs a slightly longer loop.  Measured with
+// both forced (head_dim 32 to 128, 1 to 24 segments, 1 to 256 queries, heads
+// numbered in each of the three ways, which makes no difference):
+//   K and V from HBM, a workgroup with rows for one wave: up to 5% slower at
+//   256 keys, 0-5% faster at 512, 8-15% at 1,024, 15-25% from 4,096 (none
+//   where 256 workgroups read heads of their own at head_dim 128); with rows
+//   for all waves 4-15% slower at 256, 0-8% at 512, even at 1,024, 0-8% faster
+//   at 2,048, 5-12% from 8,192 (none at head_dim 64);
+//   K and V still in the 256 MB Infinity Cache from an earlier call: even up
+//   to 1,024 keys, 4-5% slower above.
+// So the line is where a program is likely to read them from HBM: over 32 MB
+// a step through eight layers, or much else in between, has replaced them.
+// Workgroups that share a CU hide each other's waits (head_dim 64, 420
+// workgroups: 42.7 us with two stages, 43.5 with four).
+int choose_stages(const UpdateParams& p, int d, int mode, int rows, uint32_t grid, bool overlapped) {
+  if (mode != kRows || d > 2 || rows != kRowsPerBlock) return 2;
+  int64_t keys = p.segments > 1 ? 0 : p.kv_tokens;
+  for (int s = 0; p.segments > 1 && s < p.segments; ++s) keys += p.segment[s].k_len;
+  const int64_t bytes = 4 * keys * (p.q_heads / p.group) * p.head_dim;
+  const bool alone = grid <= (uint32_t)(overlapped ? kCUs / 2 : kCUs);
+  int64_t most_queries = p.segments > 1 ? 0 : p.q_tokens;
+  for (int s = 0; p.segments > 1 && s < p.segments; ++s) most_queries = std::max<int64_t>(most_queries, p.segment[s].q_len);
+  const bool one_wave = most_queries * (p.pack ? p.group : 1) <= 16;
+  const bool long_enough = keys >= int64_t(one_wave ? 512 : 1024) * std::max(1, p.segments);
+  return alone && bytes > (int64_t(32) << 20) && long_enough ? 4 : 2;
+}
+
+int padded_head_dim(int head_dim) { return head_dim <= 32 ? 0 : head_dim <= 64 ? 1 : head_dim <= 128 ? 2 : 3; }
+
+LaunchShape shape_launch(UpdateParams& p, int mode, bool overlapped) {
+  const int d = padded_head_dim(p.head_dim);
+  LaunchShape shape;
+  shape.rows = choose_rows(p, d, mode, overlapped);
+  shape.grid = number_workgroups(p, shape.rows);
+  shape.stages = choose_stages(p, d, mode, shape.rows, shape.grid, overlapped);
+  return shape;
+}
+
 hipError_t launch_update_variant(UpdateParams p, int mode, int dtype, bool overlapped, hipStream_t stream) {
-  p.cus = overlapped ? kCUs / 2 : kCUs;
-  const int d = p.head_dim <= 32 ? 0 : p.head_dim <= 64 ? 1 : p.head_dim <= 128 ? 2 : 3;
-  const int rows = choose_rows(p, d, mode, overlapped);
-  switch (d) {
-    case 0: return launch_update_d32(p, mode, rows, dtype, stream);
-    case 1: return launch_update_d64(p, mode, rows, dtype, stream);
-    case 2: return launch_update_d128(p, mode, rows, dtype, stream);
-    default: return launch_update_d256(p, mode, rows, dtype, stream);
+  const LaunchShape shape = shape_launch(p, mode, overlapped);
+  switch (padded_head_dim(p.head_dim)) {
+    case 0: return launch_update_d32(p, mode, shape, dtype, stream);
+    case 1: return launch_update_d64(p, mode, shape, dtype, stream);
+    case 2: return launch_update_d128(p, mode, shape, dtype, stream);
+    default: return launch_update_d256(p, mode, shape, dtype, stream);
   }
 }
 
@@ -582,6 +641,42 @@ int32_t scratch_on_current_device(void** address) {
 }  // namespace
 
 extern "C" {
+
+int32_t sa_update_launch_shape(const int32_t* q_tokens, const int32_t* kv_tokens, int32_t num_segments,
+                               int32_t q_heads, int32_t kv_heads, int32_t head_dim, int32_t causal_shift,
+                               int32_t causal, int32_t kv_layout, int32_t overlapped, int32_t* rows, int32_t* stages,
+                               int64_t* workgroups) {
+  sa::clear_error();
+  if (!q_tokens || !kv_tokens || num_segments < 1 || num_segments > sa::kMaxSegments || q_heads <= 0 ||
+      kv_heads <= 0 || q_heads % kv_heads != 0 || head_dim < 16 || head_dim > 256 || kv_layout < sa::kRows ||
+      kv_layout > sa::kInt8 || (kv_layout == sa::kTransposedV && head_dim != 128) ||
+      (kv_layout == sa::kInt8 && head_dim > 128) || (kv_layout != sa::kRows && num_segments > 1) || !rows || !stages ||
+      !workgroups) {
+    sa::set_error("sa_update_launch_shape: bad argument");
+    return SA_ERR_INVALID_ARGUMENT;
+  }
+  sa::UpdateParams p{};
+  p.q_heads = q_heads;
+  p.group = q_heads / kv_heads;
+  p.head_dim = head_dim;
+  p.causal = causal != 0;
+  p.causal_shift = causal_shift;
+  p.q_tokens = q_tokens[0];
+  p.kv_tokens = kv_tokens[0];
+  p.segments = num_segments > 1 ? num_segments : 0;
+  for (int32_t s = 0; s < num_segments; ++s) {
+    if (q_tokens[s] <= 0 || kv_tokens[s] < 0 || ((int64_t)q_tokens[s] + 127) / 128 * q_heads > INT32_MAX / 256) {
+      sa::set_error("sa_update_launch_shape: segment %d has bad sizes", s);
+      return SA_ERR_INVALID_ARGUMENT;
+    }
+    p.segment[s] = sa::Segment{0, 0, q_tokens[s], kv_tokens[s]};
+  }
+  const sa::LaunchShape shape = sa::shape_launch(p, kv_layout, overlapped != 0);
+  *rows = shape.rows;
+  *stages = shape.stages;
+  *workgroups = shape.grid;
+  return 0;
+}
 
 int32_t sa_run_resident_noalloc(const void* q, const void* k, const void* v, void* out, float* lse,
                                 int64_t stride_qt, int64_t stride_qh, int64_t stride_kt,

@@ -15,7 +15,8 @@
 // K/V stream through LDS in 64-key tiles, two stages: the tile after the one
 // being computed is fetched by global_load_lds_dwordx4 (HBM/L2 -> LDS with
 // no register staging) while the MFMAs run; one barrier per tile.  Small
-// launches over many keys have four stages (three tiles in flight).
+// launches over many keys have four stages, three tiles in flight
+// (choose_stages).
 //
 // v_mfma_f32_16x16x32_{bf16,f16}: A 16x32 (lane l: row l % 16, k 8 (l / 16)
 // .. +7), B 32x16 (lane l: column l % 16, k 8 (l / 16) .. +7), C 16x16 (lane
@@ -106,7 +107,6 @@ struct UpdateParams {
   int32_t numbering;      // Numbering
   int32_t slots;          // workgroups of the launch (of one XCD, for kHeadsPerXcd)
   int32_t xcd_run;        // kRunsPerXcd: ceil(slots / 8)
-  int32_t cus;            // CUs the launch has to itself (host only)
   float scale_log2;
   // INT8 K/V only: fp16 scales, element (group, kv_head) at
   // scales[group * s?s_g + kv_head * s?s_h], group = (scale_offset + key) >> scale_shift.
@@ -125,9 +125,10 @@ struct UpdateParams {
   // epilogue writes acc / l (0 where l == 0) to out and, when lse is
   // non-null, (m + log2 l) ln 2 (-inf where l == 0) to
   // lse[head * lse_sh + lse_off + query], with the expressions of
-  // finalize_kernel, and stores no state.  out may alias q: each query's
-  // row of one head is read (at the start) and written (at the end) by the
-  // same wave only.
+  // finalize_kernel, and stores no state.  out may alias q: what a wave uses
+  // of a query's row of one head it reads at the start, and only that wave
+  // writes the row, at the end.  (Lanes past the last query read the last
+  // query's row too, possibly while it is being written, and drop the value.)
   uint16_t* out;
   int64_t so_t, so_h;
   float* lse;
@@ -144,6 +145,8 @@ struct UpdateParams {
 };
 
 constexpr int kTileKeys = 64;
+constexpr int kThreads = 512;       // of a workgroup: 8 waves
+constexpr int kRowsPerBlock = 128;  // a workgroup's rows per 16-query block of its waves
 
 // The compiled variants of a padded head_dim: queries per workgroup (8 waves
 // of rows / 8), and the measured nanoseconds per 64-key tile of a workgroup
@@ -161,10 +164,17 @@ constexpr UpdateVariant kVariants[kHeadDims][kMaxVariants] = {
     {{128, 2460, 0}, {256, 3505, 0}, {0, 0, 0}},
 };
 
-// One launch with the head-dim's variant of `rows` queries per workgroup.
-hipError_t launch_update_d32(const UpdateParams&, int mode, int rows, int dtype, hipStream_t);
-hipError_t launch_update_d64(const UpdateParams&, int mode, int rows, int dtype, hipStream_t);
-hipError_t launch_update_d128(const UpdateParams&, int mode, int rows, int dtype, hipStream_t);
-hipError_t launch_update_d256(const UpdateParams&, int mode, int rows, int dtype, hipStream_t);
+// Rows of a workgroup (a variant's), LDS stages (4 only with 128 rows, V read
+// in place and head_dim up to 128) and workgroups of a launch.
+struct LaunchShape {
+  int32_t rows, stages;
+  uint32_t grid;
+};
+
+// One launch with the head-dim's variant of that shape.
+hipError_t launch_update_d32(const UpdateParams&, int mode, const LaunchShape&, int dtype, hipStream_t);
+hipError_t launch_update_d64(const UpdateParams&, int mode, const LaunchShape&, int dtype, hipStream_t);
+hipError_t launch_update_d128(const UpdateParams&, int mode, const LaunchShape&, int dtype, hipStream_t);
+hipError_t launch_update_d256(const UpdateParams&, int mode, const LaunchShape&, int dtype, hipStream_t);
 
 }  // namespace sa

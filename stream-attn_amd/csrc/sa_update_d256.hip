@@ -5,10 +5,10 @@
 
 namespace sa {
 
-hipError_t launch_update_d256(const UpdateParams& p, int mode, int rows, int dtype, hipStream_t stream) {
+hipError_t launch_update_d256(const UpdateParams& p, int mode, const LaunchShape& shape, int dtype, hipStream_t stream) {
   (void)mode;
-  return rows == 128 ? launch_variant<256, 1, kRows>(p, dtype, stream)
-                     : launch_variant<256, 2, kRows>(p, dtype, stream);
+  return shape.rows == 128 ? launch_variant<256, 1, kRows>(p, shape, dtype, stream)
+                     : launch_variant<256, 2, kRows>(p, shape, dtype, stream);
 }
 
 }  // namespace sa

@@ -2,7 +2,6 @@
 // included by the sources that compile one head-dim's variants.
 #pragma once
 
-#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -251,14 +250,14 @@ struct Geometry {
 // key 16 ((s >> 2) & 1) + 4 (s >> 3) + (s & 3)), zero keys up to a multiple
 // of 64.
 // STAGES: LDS stages, of which all but one are in flight while a tile is
-// computed (2, or a power of two above it for V read in place).
+// computed (2, or 4 for V read in place).
 template <typename Op, int DP, int QB, int MODE, int STAGES>
 __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const UpdateParams p) {
   using Geo = Geometry<DP>;
   constexpr bool VT = MODE == kTransposedV;
   constexpr bool QUANT = MODE == kInt8;
   constexpr bool RING = STAGES > 2;
-  static_assert(!RING || (MODE == kRows && (STAGES & (STAGES - 1)) == 0), "ring of stages");
+  static_assert(STAGES == 2 || (STAGES == 4 && MODE == kRows), "LDS stages");
   constexpr int CK = Geo::CK;
   constexpr int DB = Geo::DB;
   // Fragments read before one wait: KB 32-wide d steps of K (two fragments
@@ -659,7 +658,6 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
     // tile t is there once no more than the later tiles' are outstanding.
     constexpr int PER_TILE = 2 * Geo::PIECES / Geo::ISSUERS;
     static_assert((STAGES - 2) * PER_TILE <= 63, "vmcnt range");
-    static_assert(STAGES == 4, "waits below");
     for (int t = 0; t < ntiles; ++t) {
       const int later = ntiles - 1 - t;
       if (later >= 2)
@@ -842,50 +840,22 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
 }
 
 template <typename Op, int DP, int QB, int MODE>
-hipError_t launch_kernel(UpdateParams p, hipStream_t stream) {
-  constexpr int rows = Geometry<DP>::WAVES * 16 * QB;
-  const bool several = p.segments > 1;
-  int64_t most_queries = several ? 0 : p.q_tokens;
-  for (int s = 0; several && s < p.segments; ++s) most_queries = std::max<int64_t>(most_queries, p.segment[s].q_len);
-  p.pack = QB == 1 && p.group > 1 && most_queries * p.group <= INT32_MAX;
-  p.unit_heads = p.pack ? p.q_heads / p.group : p.q_heads;
-  p.numbering = p.unit_heads % 8 == 0 ? kHeadsPerXcd : p.causal || several ? kDealt : kRunsPerXcd;
-  const int heads = p.numbering == kHeadsPerXcd ? p.unit_heads / 8 : p.unit_heads;
-  const int per_query = p.pack ? p.group : 1;
-  p.slots = 0;
-  [[maybe_unused]] int64_t keys = several ? 0 : p.kv_tokens;
-  for (int s = 0; s < (several ? p.segments : 1); ++s) {
-    if (several) keys += p.segment[s].k_len;
-    p.first[s] = p.slots;
-    const int64_t queries = several ? p.segment[s].q_len : p.q_tokens;
-    p.slots += (int32_t)((queries * per_query + rows - 1) / rows * heads);
-  }
-  p.xcd_run = (p.slots + 7) / 8;
-  const unsigned grid = p.numbering == kHeadsPerXcd ? 8u * p.slots : p.numbering == kDealt ? p.slots : 8u * p.xcd_run;
+hipError_t launch_kernel(const UpdateParams& p, const LaunchShape& shape, hipStream_t stream) {
   if constexpr (QB == 1 && MODE == kRows && DP <= 128) {
-    // Workgroups that have a CU to themselves have the LDS for two more tiles
-    // in flight, where two stages waited for HBM at every barrier (head_dim
-    // 128, 24 decoding sequences of 8,000 keys, 786 MB of K and V, 272 -> 235
-    // us; 1,009 queries over 61,312 keys, 251 MB, 1,137 -> 1,040 us).  K and V
-    // that the XCDs' L2 (4 MB each) hold come back soon enough, and two
-    // workgroups on a CU hide each other's waits: there the ring's longer
-    // start and loop took 5% (2,476 x 8 heads, 10 MB) and 2% (head_dim 64,
-    // 420 workgroups) more.
-    constexpr int64_t kL2Bytes = int64_t(8 * 4) << 20;
-    const int64_t workgroups = (int64_t)p.slots * (p.numbering == kHeadsPerXcd ? 8 : 1);
-    if (workgroups <= p.cus && 4 * keys * (p.q_heads / p.group) * p.head_dim > kL2Bytes) {
-      hipLaunchKernelGGL((update_kernel<Op, DP, QB, MODE, 4>), dim3(grid), dim3(Geometry<DP>::THREADS), 0, stream, p);
+    if (shape.stages == 4) {
+      hipLaunchKernelGGL((update_kernel<Op, DP, QB, MODE, 4>), dim3(shape.grid), dim3(Geometry<DP>::THREADS), 0, stream, p);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((update_kernel<Op, DP, QB, MODE, 2>), dim3(grid), dim3(Geometry<DP>::THREADS), 0, stream, p);
+  hipLaunchKernelGGL((update_kernel<Op, DP, QB, MODE, 2>), dim3(shape.grid), dim3(Geometry<DP>::THREADS), 0, stream, p);
   return hipGetLastError();
 }
 
 template <int DP, int QB, int MODE>
-hipError_t launch_variant(const UpdateParams& p, int dtype, hipStream_t stream) {
-  return dtype == SA_DTYPE_BF16 ? launch_kernel<BF16, DP, QB, MODE>(p, stream)
-                                : launch_kernel<FP16, DP, QB, MODE>(p, stream);
+hipError_t launch_variant(const UpdateParams& p, const LaunchShape& shape, int dtype, hipStream_t stream) {
+  static_assert(Geometry<DP>::THREADS == kThreads && Geometry<DP>::WAVES * 16 == kRowsPerBlock, "launch shape");
+  return dtype == SA_DTYPE_BF16 ? launch_kernel<BF16, DP, QB, MODE>(p, shape, stream)
+                                : launch_kernel<FP16, DP, QB, MODE>(p, shape, stream);
 }
 
 }  // namespace

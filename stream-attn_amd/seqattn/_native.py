@@ -58,6 +58,10 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         + [c_int32] * 9
         + [c_double, c_int32, c_int32, c_int32, c_void_p],
     ),
+    "sa_update_launch_shape": (
+        c_int32,
+        [ctypes.POINTER(c_int32)] * 2 + [c_int32] * 8 + [ctypes.POINTER(c_int32)] * 2 + [ctypes.POINTER(c_int64)],
+    ),
     "sa_finalize_attention": (
         c_int32,
         [c_void_p] * 5 + [c_int64] * 8 + [c_int32] * 4 + [c_void_p],

@@ -152,6 +152,44 @@ def test_noalloc_entry_point_rejects_bad_arguments_before_touching_the_gpu():
     assert b"segment 1 needs" in message and b"67108864" in message
 
 
+@pytest.mark.skipif(not _native.library_is_built(), reason="native library not built")
+def test_update_launch_shape():
+    import ctypes
+
+    lib = _native.lib()
+
+    def shape(q, k, heads, head_dim, *, causal=1, kv_layout=0, overlapped=0):
+        arrays = [(ctypes.c_int32 * len(x))(*x) for x in (q, k)]
+        rows, stages, workgroups = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int64()
+        status = lib.sa_update_launch_shape(*arrays, len(q), *heads, head_dim, k[0] - q[0], causal, kv_layout,
+                                            overlapped, rows, stages, workgroups)
+        return (rows.value, stages.value, workgroups.value) if status == 0 else status
+
+    gqa, mha = (32, 8), (8, 8)
+    # Decoding: the 4 query heads of a K/V head share a workgroup.
+    assert shape([1] * 24, [8000] * 24, gqa, 128) == (128, 4, 192)
+    assert shape([1009], [61312], gqa, 128) == (128, 4, 256)
+    assert shape([65536], [65536], (32, 32), 128, causal=0)[:2] == (384, 2)
+    # Four stages: K and V over 32 MB (8,192 keys x 8 heads x d128 are 32 MB) ...
+    assert [shape([1], [n], gqa, 128)[1] for n in (8192, 8193)] == [2, 4]
+    # ... of at least 512 keys a segment on average, 1,024 where a workgroup
+    # has rows for more than one wave ...
+    assert [shape([4] * 17, [512] * 16 + [m], gqa, 128)[1] for m in (511, 512)] == [2, 4]
+    assert [shape([4] * 16 + [5], [1024] * 16 + [m], gqa, 128)[1] for m in (1023, 1024)] == [2, 4]
+    # ... by workgroups with a CU each (half the chip beside another launch) ...
+    assert [shape([1] * n, [4000] * n, mha, 128)[1:] for n in (32,)] == [(4, 256)]
+    assert [shape([n], [20000], (33, 33), 128, causal=0)[1:] for n in (800, 900)] == [(4, 232), (2, 264)]
+    assert [shape([1] * n, [4000] * n, mha, 128, overlapped=1)[1] for n in (16, 17)] == [4, 2]
+    # ... for 16-bit K and V up to head_dim 128.
+    assert [shape([1], [80000], gqa, d)[1] for d in (16, 96, 128, 136)] == [4, 4, 4, 2]
+    assert shape([1], [20000], gqa, 128, kv_layout=2)[1] == 2
+    for bad in (dict(q=[1], k=[5], heads=(6, 4), head_dim=64), dict(q=[1] * 33, k=[5] * 33, heads=gqa, head_dim=64),
+                dict(q=[0], k=[5], heads=gqa, head_dim=64), dict(q=[1], k=[5], heads=gqa, head_dim=64, kv_layout=1),
+                dict(q=[1], k=[5], heads=gqa, head_dim=136, kv_layout=2),
+                dict(q=[1, 1], k=[5, 5], heads=gqa, head_dim=128, kv_layout=2)):
+        assert shape(**bad) == -1
+
+
 PROBE_HEADER = HEADER.parent / "seqattn_probe.h"
 PROBE_LIB = Path(_native.LIB_PATH).parent / "libseqattn_probe.so"
 
