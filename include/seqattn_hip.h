@@ -469,8 +469,11 @@ int32_t sa_pipeline_attach_resident_scratch(sa_pipeline* pipeline, void* scratch
 /*
  * The scratch bytes that sa_pipeline_run_resident would use for these segments,
  * V's token stride and this output (strides as there): the largest of the
- * copies it makes, 0 when it reads V in place.  Host arithmetic only.
+ * copies it makes, 0 when it reads V in place.  Host arithmetic only.  With V's
+ * token stride in [1, 2^24) no segment of fewer than sa_resident_copy_rows()
+ * queries x query heads per K/V head makes one.
  */
+int32_t sa_resident_copy_rows(void);
 int32_t sa_pipeline_resident_scratch_bytes(
     sa_pipeline* pipeline, int64_t stride_vt, const void* out, int64_t stride_ot, int64_t stride_oh,
     const int64_t* cu_seqlens_q, const int64_t* cu_seqlens_k, int32_t num_segments, int64_t* bytes);

@@ -85,8 +85,9 @@ struct SegmentGroup {
 // no gain at 32,768, 2-8% slower at 8,192 and below, where it also cannot
 // join a launch with other segments.  V read in place needs a token stride in
 // [1, 2^24) (32-bit offsets within a tile); the copy reads any.
+constexpr int32_t kTransposeRows = 65536;
 inline bool transposes_v(int64_t q_length, int64_t group, int64_t sv_t) {
-  return q_length * group >= 65536 || sv_t <= 0 || sv_t >= (1 << 24);
+  return q_length * group >= kTransposeRows || sv_t <= 0 || sv_t >= (1 << 24);
 }
 }  // namespace sa
 

@@ -1918,6 +1918,8 @@ int32_t sa_pipeline_run_resident(sa_pipeline* p, const void* q, const void* k, c
   return sa::exception_status("sa_pipeline_run_resident", error);
 }
 
+int32_t sa_resident_copy_rows(void) { return sa::kTransposeRows; }
+
 int32_t sa_pipeline_resident_scratch_bytes(sa_pipeline* p, int64_t stride_vt, const void* out, int64_t stride_ot,
                                            int64_t stride_oh, const int64_t* cu_seqlens_q,
                                            const int64_t* cu_seqlens_k, int32_t num_segments, int64_t* bytes) {

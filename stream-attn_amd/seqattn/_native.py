@@ -144,6 +144,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     ),
     "sa_pipeline_synchronize": (c_int32, [c_void_p]),
     "sa_pipeline_attach_resident_scratch": (c_int32, [c_void_p, c_void_p, c_int64]),
+    "sa_resident_copy_rows": (c_int32, []),
     "sa_pipeline_resident_scratch_bytes": (
         c_int32,
         [c_void_p, c_int64, c_void_p, c_int64, c_int64, ctypes.POINTER(c_int64), ctypes.POINTER(c_int64), c_int32,

@@ -148,7 +148,8 @@ class HipExecutorMixin:
         compute = workspace.compute_stream
         bounds = (_bounds_array(q_bounds), _bounds_array(k_bounds), len(q_bounds) - 1)
         stats.resident_scratch_bytes = 0
-        if self.plan.head_dim == 128:
+        if self.plan.head_dim == 128 and (q.shape[0] >= workspace.resident_copy_queries
+                                          or not 0 < v.stride(0) < 1 << 24):
             needed = ctypes.c_int64()
             status = _native.lib().sa_pipeline_resident_scratch_bytes(
                 workspace.handle, v.stride(0), out.data_ptr(), *out.stride()[:2], *bounds, ctypes.byref(needed)

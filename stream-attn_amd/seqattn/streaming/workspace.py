@@ -87,6 +87,8 @@ class CudaWorkspace:
         self._lib = _native.lib()
         self.plan = plan
         self.resident_scratch: torch.Tensor | None = None
+        # Queries from which a segment of a resident run may read V through a copy.
+        self.resident_copy_queries = -(-self._lib.sa_resident_copy_rows() * plan.kv_heads // plan.q_heads)
         self.host_staging: torch.Tensor | None = None
         self._staging_attached = False
         if plan.schedule == "head_groups":

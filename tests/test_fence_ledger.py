@@ -45,7 +45,7 @@ def ledger(tmp_path_factory):
     subprocess.run(cmd, check=True, capture_output=True)
     lib = ctypes.CDLL(str(out))
     for name, (restype, argtypes) in _native.SIGNATURES.items():
-        if name.startswith("sa_pipeline") or name in ("sa_last_error", "sa_abi_version"):
+        if name.startswith("sa_pipeline") or name in ("sa_last_error", "sa_abi_version", "sa_resident_copy_rows"):
             fn = getattr(lib, name)
             fn.restype, fn.argtypes = restype, argtypes
     lib.ledger_check.restype = ctypes.c_int64
@@ -823,6 +823,8 @@ def test_resident_scratch_is_what_the_run_reads(ledger, q_lengths, k_lengths, he
     assert ledger.sa_pipeline_resident_scratch_bytes(p.handle, stride_vt, out, *qs, cu_q, cu_k, len(q_lengths),
                                                      ctypes.byref(needed)) == 0
     assert needed.value == kv_heads * 128 * (-(-longest // 64) * 64) * HEAD_BYTES
+    if 0 < stride_vt < 1 << 24 and max(q_lengths) * q_heads // kv_heads < ledger.sa_resident_copy_rows():
+        assert needed.value == 0
 
     def launches(scratch_bytes):
         ledger.ledger_reset()
