@@ -267,7 +267,11 @@ LaunchShape shape_launch(UpdateParams& p, int mode, bool overlapped) {
   return shape;
 }
 
-hipError_t launch_update_variant(UpdateParams p, int mode, int dtype, bool overlapped, hipStream_t stream) {
+// A launch has fewer than 2^32 threads (numbering rounds its workgroups up by
+// at most 7).
+constexpr int64_t kMaxWorkgroups = (int64_t(1) << 32) / kThreads - 8;
+
+hipError_t launch_one(UpdateParams p, int mode, int dtype, bool overlapped, hipStream_t stream) {
   const LaunchShape shape = shape_launch(p, mode, overlapped);
   switch (padded_head_dim(p.head_dim)) {
     case 0: return launch_update_d32(p, mode, shape, dtype, stream);
@@ -275,6 +279,31 @@ hipError_t launch_update_variant(UpdateParams p, int mode, int dtype, bool overl
     case 2: return launch_update_d128(p, mode, shape, dtype, stream);
     default: return launch_update_d256(p, mode, shape, dtype, stream);
   }
+}
+
+// More queries than one launch's workgroups hold go in several launches of
+// consecutive rows (a query's bits do not depend on its neighbours).
+hipError_t launch_update_variant(UpdateParams p, int mode, int dtype, bool overlapped, hipStream_t stream) {
+  // A common multiple of the widths and of the state's 16-row groups.
+  constexpr int64_t kStep = 768;
+  const int64_t most = (kMaxWorkgroups / p.q_heads - 1) * kRowsPerBlock / kStep * kStep;
+  while (p.segments <= 1 && most > 0 && p.q_tokens > most) {
+    UpdateParams part = p;
+    part.q_tokens = (int32_t)most;
+    const hipError_t err = launch_one(part, mode, dtype, overlapped, stream);
+    if (err != hipSuccess) return err;
+    p.q += most * p.sq_t;
+    p.q_local_offset += (int32_t)most;
+    p.q_tokens -= (int32_t)most;
+    if (p.out != nullptr) p.out += most * p.so_t;
+    p.lse_off += most;
+    if (p.m != nullptr) {
+      p.m += most * (p.tiled_state ? p.q_heads : p.ss_t);
+      p.l += most * (p.tiled_state ? p.q_heads : p.ss_t);
+      p.acc += most * (p.tiled_state ? (int64_t)p.q_heads * p.head_dim : p.sa_t);
+    }
+  }
+  return launch_one(p, mode, dtype, overlapped, stream);
 }
 
 // The segments of one call in launches of up to kMaxSegments, those with the
@@ -288,13 +317,12 @@ int32_t launch_segments(UpdateParams p, const FusedOutput& fused, int dtype, boo
   for (int32_t s = 0; s < fused.num_segments; ++s)
     if (fused.segments[s].q_len > 0) order.push_back(fused.segments[s]);
   std::stable_sort(order.begin(), order.end(), [](const Segment& a, const Segment& b) { return a.k_len > b.k_len; });
-  const int64_t most = (int64_t)INT32_MAX / 8;  // workgroups of a launch
   for (size_t at = 0; at < order.size();) {
     int64_t workgroups = 0;
     p.segments = 0;
     while (at < order.size() && p.segments < kMaxSegments) {
       const int64_t more = ((int64_t)order[at].q_len + 127) / 128 * p.q_heads;
-      if (p.segments > 0 && workgroups + more > most) break;
+      if (p.segments > 0 && workgroups + more > kMaxWorkgroups) break;
       workgroups += more;
       p.segment[p.segments++] = order[at++];
     }

@@ -78,3 +78,33 @@ def test_broadcast_v_rows_are_read_through_the_transposed_copy():
     torch.cuda.synchronize()
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("rows,count", [(1_200_000_000, 1), (34_000_000, 34)])
+def test_more_queries_than_one_launch_holds(rows, count):
+    """2.4e9 and 2.3e9 query x head pairs at head_dim 16: more than a launch's
+    2^32 threads, in one segment and over segments.  Every query is the same
+    row (token stride 0), so every output row is that of a small run."""
+    print(f"[gpu case] segments of {rows} x {count} queries", flush=True)
+    heads, d, keys = 2, 16, 64
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    q, k, v = (torch.randn((n, heads, d), generator=gen, device="cuda").to(torch.bfloat16) for n in (1, keys, keys))
+    config = StreamingAttentionConfig(kv_chunk_tokens=64)
+    plan = build_plan(q_heads=heads, kv_heads=heads, head_dim=d, dtype=torch.bfloat16, device="cuda", max_q_tokens=256,
+                      max_kv_tokens=keys * count, config=config)
+    runner = StreamingAttentionRunner(plan, config)
+    expected = runner(q, k, v, torch.tensor([0, 1]), torch.tensor([0, keys]))
+    total = rows * count
+    out = torch.empty((total, heads, d), dtype=torch.bfloat16, device="cuda")
+    k_all, v_all = (x.repeat(count, 1, 1) for x in (k, v))
+    cu_q, cu_k = ((ctypes.c_int64 * (count + 1))(*range(0, n * count + 1, n)) for n in (rows, keys))
+    workspace = runner._workspace
+    _native.check(_native.lib().sa_pipeline_run_resident(
+        workspace.handle, q.data_ptr(), k_all.data_ptr(), v_all.data_ptr(), out.data_ptr(), None, 0, d, heads * d, d,
+        heads * d, d, heads * d, d, 0, cu_q, cu_k, count, d**-0.5, 0, workspace.compute_stream.cuda_stream, None),
+        "sa_pipeline_run_resident")
+    step = 50_000_000
+    for start in range(0, total, step):
+        assert bool((out[start:start + step] == expected).all()), start
+    torch.cuda.synchronize()
+    runner.close()
