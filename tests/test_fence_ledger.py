@@ -363,11 +363,13 @@ def test_head_group_schedule_is_race_free(ledger, num_sets, causal, heads):
 @pytest.mark.parametrize("num_sets", [1, 2])
 def test_head_group_schedule_with_transposed_v_is_race_free(ledger, num_sets):
     ledger.ledger_reset()
-    run_head_groups(ledger, num_sets=num_sets, causal=True, q_lengths=[700, 0, 1900], k_lengths=[900, 40, 1300],
-                    group_kv=1, q_heads=8, kv_heads=4, head_dim=128, with_vt=True)
+    # Two segments of 65,536 queries x query heads per K/V head and more, and
+    # one that reads V in place.
+    run_head_groups(ledger, num_sets=num_sets, causal=True, q_lengths=[32768, 0, 32767, 35000],
+                    k_lengths=[900, 40, 700, 1300], group_kv=1, q_heads=8, kv_heads=4, head_dim=128, with_vt=True)
     counts = (ctypes.c_int64 * 4)()
     ledger.ledger_counts(counts)
-    assert counts[2] == 4 * 2 * 2  # per unit and non-empty segment: a transpose and an update launch
+    assert counts[2] == 4 * (2 + 1 + 2)  # per unit: an update launch a segment, a transpose before two of them
     check(ledger, f"head groups with transposed V, sets={num_sets}")
 
 

@@ -6,10 +6,11 @@ launch per (unit, segment).  Its output and LSE must equal the default
 Q-block schedule's bit for bit for the same K/V chunk (the row sums merge at
 the same boundaries), and match the FP32 oracle within the tolerances of
 tests/test_gpu_streaming.py.  Layouts are forced through the plan (K/V heads
-per unit, one or two buffer sets, transposed V or V read in place) so that
-every path of the schedule runs: units that alternate streams, a short last
-unit, a single unit holding every head, empty and ragged segments, GQA,
-causal masks with rows that see no key, fp16, and the 32-query kernel.
+per unit, one or two buffer sets, with and without space for V transposed) so
+that every path of the schedule runs: units that alternate streams, a short
+last unit, a single unit holding every head, empty and ragged segments, GQA,
+causal masks with rows that see no key, fp16, other head_dims, and segments of
+enough queries to read V through its transposed copy.
 """
 
 from __future__ import annotations
@@ -46,14 +47,14 @@ def head_group_plan(q, k, config, *, group_kv, sets, transposed_v):
 
 
 CASES = [
-    # (dtype, head_dim, q_heads, kv_heads, K/V heads per unit, sets, transposed V)
+    # (dtype, head_dim, q_heads, kv_heads, K/V heads per unit, sets, space for V transposed)
     (torch.bfloat16, 128, 4, 4, 1, 2, True),    # one head per unit, units alternate streams
     (torch.bfloat16, 128, 4, 4, 3, 1, False),   # one set, a short last unit
     (torch.bfloat16, 128, 4, 4, 4, 2, True),    # a single unit holds every head
     (torch.bfloat16, 128, 8, 2, 1, 2, False),   # GQA, V read in place
     (torch.float16, 128, 6, 3, 2, 2, True),     # fp16, GQA, short last unit
-    (torch.bfloat16, 96, 4, 2, 1, 2, False),    # a partial d block of the 48-query kernel
-    (torch.bfloat16, 64, 6, 3, 2, 1, False),    # the 32-query kernel
+    (torch.bfloat16, 96, 4, 2, 1, 2, False),    # a partial d step
+    (torch.bfloat16, 64, 6, 3, 2, 1, False),    # a padded head_dim of 64
 ]
 
 
@@ -88,6 +89,30 @@ def test_head_groups_bit_identical_to_q_blocks(case, causal):
     assert st_h.max_resident_q_tokens == 2500
     ref_o, ref_l = oracle(q, k, v, cu_q, cu_k, q_chunk=512, kv_chunk=256, causal=causal)
     check(out_h, lse_h, ref_o, ref_l)
+
+
+@pytest.mark.parametrize("sets", [1, 2])
+@pytest.mark.parametrize("causal", [False, True])
+def test_head_groups_read_v_of_large_segments_through_its_copy(causal, sets):
+    """From 65,536 queries x query heads per K/V head a segment reads V
+    transposed, the two around it here; with no space for the copy, or in Q
+    blocks, it reads V in place: the same bits."""
+    announce(f"head groups transposed V sets={sets} causal={causal}")
+    gen = torch.Generator().manual_seed(53)
+    cu_q = torch.tensor([0, 2048, 2148, 4248], dtype=torch.int32)
+    cu_k = torch.tensor([0, 2111, 2400, 3533], dtype=torch.int32)
+    q = pinned_randn((4248, 64, 128), torch.bfloat16, gen)
+    k, v = (pinned_randn((3533, 2, 128), torch.bfloat16, gen) for _ in range(2))
+    config = StreamingAttentionConfig(backend="hip", q_chunk_tokens=2048, kv_chunk_tokens=512)
+    base = build_plan(q_heads=64, kv_heads=2, head_dim=128, dtype=torch.bfloat16, device="cuda", max_q_tokens=4248,
+                      max_kv_tokens=3533, config=config)
+    results = [run_plan(base, config, q, k, v, cu_q, cu_k, causal)]
+    for transposed_v in (True, False):
+        plan = head_group_plan(q, k, config, group_kv=1, sets=sets, transposed_v=transposed_v)
+        results.append(run_plan(plan, dataclasses.replace(config, schedule="head_groups"), q, k, v, cu_q, cu_k, causal))
+    for out, lse, _ in results[1:]:
+        assert torch.equal(out, results[0][0])
+        assert torch.equal(lse, results[0][1])
 
 
 def test_head_groups_repeated_runs_reuse_the_sets():
