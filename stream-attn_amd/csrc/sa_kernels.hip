@@ -141,8 +141,8 @@ int64_t tiles_of(int64_t keys) { return (std::max<int64_t>(0, keys) + kTileKeys 
 // run in rounds of one (or two) workgroups per CU; under a causal mask and
 // with several segments long blocks start first and short ones fill in behind
 // them, and a launch that shares the chip with another one fills in behind
-// that.  No launch ends before its longest block.  Over 60 drawn shapes the
-// choice was within 3% of the best variant's time on average.
+// that.  No launch ends before its longest block.  Over 60 drawn launches the
+// chosen width took 0.8% more than the best one on average, 6.7% at most.
 double variant_time(const UpdateVariant& v, const UpdateParams& p, bool overlapped) {
   // The narrowest workgroups pack the query heads of a K/V head.
   const int64_t group = v.rows == kVariants[0][0].rows ? p.group : 1;
@@ -184,7 +184,7 @@ double variant_time(const UpdateVariant& v, const UpdateParams& p, bool overlapp
 
 // Queries per workgroup.  A query's bits do not depend on it, so it is chosen
 // for time alone: wide workgroups read each K/V tile for more queries (bf16,
-// head_dim 128: 6.7 ns per query and tile at 384 queries, 7.8 at 128), narrow
+// head_dim 128: 6.1 ns per query and tile at 384 queries, 7.6 at 128), narrow
 // ones fill the chip with few queries and waste less of a last round or of a
 // causal diagonal.  1,009 queries over 61,312 keys x 32 heads: 384 queries
 // are 96 workgroups, 128 are 256.
@@ -232,13 +232,13 @@ uint32_t number_workgroups(UpdateParams& p, int rows) {
 // in flight, but starts later and runs a slightly longer loop.  Measured with
 // both forced (head_dim 32 to 128, 1 to 24 segments, 1 to 256 queries, heads
 // numbered in each of the three ways, which makes no difference):
-//   K and V from HBM, a workgroup with rows for one wave: up to 5% slower at
-//   256 keys, 0-5% faster at 512, 8-15% at 1,024, 15-25% from 4,096 (none
-//   where 256 workgroups read heads of their own at head_dim 128); with rows
-//   for all waves 4-15% slower at 256, 0-8% at 512, even at 1,024, 0-8% faster
-//   at 2,048, 5-12% from 8,192 (none at head_dim 64);
-//   K and V still in the 256 MB Infinity Cache from an earlier call: even up
-//   to 1,024 keys, 4-5% slower above.
+//   K and V from HBM, time with four over two stages.  Rows for one wave: 0.99
+//   to 1.05 at 256 keys, 0.91-1.0 at 512, 0.84-0.94 at 1,024, 0.71-0.91 from
+//   4,096 (1.0 where 256 workgroups read heads of their own).  Rows for all
+//   waves: 1.03-1.15 at 256, 1.0-1.1 at 512, 0.96-1.05 at 1,024, 0.90-1.04 at
+//   2,048, 0.85-1.0 from 8,192.
+//   K and V still in the 256 MB Infinity Cache from an earlier call: 0.99-1.06
+//   at 1,024 keys, 1.02-1.09 above.
 // So the line is where a program is likely to read them from HBM: over 32 MB
 // a step through eight layers, or much else in between, has replaced them.
 // Workgroups that share a CU hide each other's waits (head_dim 64, 420

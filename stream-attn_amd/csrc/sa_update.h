@@ -151,7 +151,10 @@ constexpr int kRowsPerBlock = 128;  // a workgroup's rows per 16-query block of 
 // The compiled variants of a padded head_dim: queries per workgroup (8 waves
 // of rows / 8), and the measured nanoseconds per 64-key tile of a workgroup
 // alone on its CU (`one`) and of two workgroups sharing a CU (`two`, 0 where
-// registers or LDS hold one): bf16, V read in place, 256 CUs busy.
+// registers or LDS hold one): bf16, V read in place, 256 CUs busy.  The present
+// build on another box takes 4-16% less throughout; with those figures 58 drawn
+// launches choose the same widths.  (Up to four head_dim-32 workgroups fit on a
+// CU; the model counts two.)
 struct UpdateVariant {
   int32_t rows, one, two;
 };

@@ -80,7 +80,8 @@ __device__ inline u32x4 q_sign(float scale_log2) {
 // cannot relate an LDS read to the DMA writing the other stage and would wait
 // for that prefetch (vmcnt) before it, and because its own schedule waited
 // three times per step (with the second wave of the SIMD usually waiting at
-// the same moment).
+// the same moment); plain loads and the transposing builtin at head_dim 256
+// took 2-14% more.
 
 // w[kb N / 2 + c] = the 16 bytes at addr + base + kb * step + c KB.
 template <int N>
@@ -261,11 +262,13 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
   constexpr int CK = Geo::CK;
   constexpr int DB = Geo::DB;
   // Fragments read before one wait: KB 32-wide d steps of K (two fragments
-  // each) and VB d blocks of V, as many as the registers hold.  Measured per
-  // 64-key tile with one workgroup on every CU: head_dim 256, 32 queries per
-  // wave, 3.4 us with (2, 4) and 3.9 us with (2, 2); 16 queries 2.3 us with
-  // (4, 8).  head_dim 128, 48 queries on a full chip: 2.45 us with VB 8, 2.50
-  // with 2.
+  // each) and VB d blocks of V, as many as the registers hold.  Measured:
+  // head_dim 256, 32 queries per wave, 9,239 x 16 heads 1,350 us with (2, 4),
+  // 1,379 with (2, 2) or (1, 4), more with spills above; 16 queries, 200 over
+  // 20,000 keys x 16 heads 703 us with (4, 8), 722 with (4, 4), 735 with (2, 8).
+  // head_dim 128, 48 queries per wave 2.45 us a tile on a full chip with VB 8,
+  // 2.50 with 2; 16 queries with INT8 K/V 243 us with VB 4, 249 with 8 (667
+  // queries over 8,446 keys x 40/8 heads).
   constexpr int KB = DP == 256 ? (QB == 1 ? 4 : 2) : CK;
   constexpr int VB = DP == 256 ? (QB == 1 ? 8 : 4) : DP == 32 ? 2 : DP == 128 && QB > 1 ? 8 : 4;
   constexpr int BLOCK_M = Geo::WAVES * 16 * QB;

@@ -144,7 +144,7 @@ def run_tensor_mode(lib, *, num_kv, num_out, causal, q_lengths, k_lengths, q_chu
 
 CASES = [
     # (q segment lengths, k segment lengths): several passes per segment, a
-    # Q block above 512 rows (split launches), a short last pass, ragged chunks.
+    # Q block of 512 rows and more (split launches at head_dim 64), a short last pass, ragged chunks.
     ([3000, 700], [2600, 900]),
     ([1500], [1500]),
     ([200, 0, 3100], [500, 300, 2049]),

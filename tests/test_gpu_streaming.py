@@ -98,9 +98,8 @@ def test_matches_oracle_at_reference_test_shapes(dtype, causal, q_heads, kv_head
     check(out, lse, ref_o, ref_l)
 
 
-# Every kernel geometry and its edges: the 32-query kernel at head_dim 16-64
-# and 136-256, the 48-query kernel at 72-128, including head_dims that end
-# inside a 16-wide d block (40, 72, 104, 120) or a 32-wide d step (80).
+# Every padded head_dim (32, 64, 128, 256) and its edges, including head_dims
+# that end inside a 16-wide d block (40, 72, 104, 120) or a 32-wide d step (80).
 @pytest.mark.parametrize("head_dim", [16, 32, 40, 48, 64, 72, 80, 96, 104, 120, 128, 136, 200, 256])
 @pytest.mark.parametrize("causal", [False, True])
 def test_head_dims_ragged_chunks(head_dim, causal):
@@ -340,8 +339,9 @@ def test_transposed_v_pads_short_segments_exactly(causal):
 @pytest.mark.parametrize("num_kv", [1, 3])
 @pytest.mark.parametrize("causal", [False, True])
 def test_split_chunk_updates_on_two_streams_are_bit_identical(causal, num_kv):
-    """Streamed Q blocks of 512 rows or more apply each K/V chunk with two
-    launches, one per half of the rows, on two streams.  With a one-slot ring
+    """Streamed Q blocks of two workgroup tiles or more (768 rows at head_dim
+    128) apply each K/V chunk with two launches, one per half of the rows, on
+    two streams.  With a one-slot ring
     the next copy must wait for both halves; with three slots the halves run
     ahead of each other.  Host output, device-consumer output and the
     HBM-resident single launch agree bit for bit."""
