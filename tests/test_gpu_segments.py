@@ -108,3 +108,5 @@ def test_more_queries_than_one_launch_holds(rows, count):
         assert bool((out[start:start + step] == expected).all()), start
     torch.cuda.synchronize()
     runner.close()
+    del out
+    torch.cuda.empty_cache()  # 70 GB and more
