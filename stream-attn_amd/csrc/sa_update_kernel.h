@@ -267,9 +267,10 @@ __global__ __launch_bounds__(Geometry<DP>::THREADS) void update_kernel(const Upd
   // 1,379 with (2, 2) or (1, 4), more with spills above; 16 queries, 200 over
   // 20,000 keys x 16 heads 703 us with (4, 8), 722 with (4, 4), 735 with (2, 8).
   // head_dim 128, 48 queries per wave 2.45 us a tile on a full chip with VB 8,
-  // 2.50 with 2; 16 queries with INT8 K/V 243 us with VB 4, 249 with 8 (667
-  // queries over 8,446 keys x 40/8 heads).
-  constexpr int KB = DP == 256 ? (QB == 1 ? 4 : 2) : CK;
+  // 2.50 with 2; 16 queries, 1,009 over 61,312 keys x 32/8 heads 1,058 us with
+  // (4, 4), 1,071 with (2, 4) or (4, 8), and with INT8 K/V, 667 over 8,446 keys
+  // x 40/8 heads, 240 us with (2, 4), 243 with (4, 4), 249 with (4, 8).
+  constexpr int KB = DP == 256 ? (QB == 1 ? 4 : 2) : DP == 128 && QUANT && QB == 1 ? 2 : CK;
   constexpr int VB = DP == 256 ? (QB == 1 ? 8 : 4) : DP == 32 ? 2 : DP == 128 && QB > 1 ? 8 : 4;
   constexpr int BLOCK_M = Geo::WAVES * 16 * QB;
   static_assert(!QUANT || (Geo::I8_DMAS <= Geo::WAVES && Geo::I8_GRANULES <= Geo::THREADS), "INT8 staging");
