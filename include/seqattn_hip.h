@@ -321,9 +321,9 @@ int32_t sa_pipeline_run(
  * output copy is made.  Enqueued on compute_stream (and the pipeline's
  * second stream, joined back into it); returns once the host inputs have
  * been copied, before the launches end: later work on compute_stream sees
- * the output and the LSE.  An error return waits as sa_pipeline_run's does.  No counterpart in
- * the reference (its device outputs go through output_transform,
- * executor.py:145-172).
+ * the output and the LSE.  An error return waits as sa_pipeline_run's does.
+ * No counterpart in the reference (its device outputs go through
+ * output_transform, executor.py:145-172).
  */
 int32_t sa_pipeline_run_device_output(
     sa_pipeline* pipeline,

@@ -82,9 +82,10 @@ struct SegmentGroup {
 // there is scratch for one).  The copy moves V twice, one launch of its own;
 // its fragments then take half the LDS instructions.  Measured with head_dim
 // 128, 8/8, 32/8 and 32/32 heads: 0.2-1.3% faster at 65,536 and more queries x
-// query heads per K/V head, 0.8% faster to even at 32,768, 2-6% slower at 8,192
-// and up to 28% below, where it also cannot join a launch with other segments.  V read in place needs a token stride in
-// [1, 2^24) (32-bit offsets within a tile); the copy reads any.
+// query heads per K/V head, even to 0.8% faster at 32,768, 2-6% slower at 8,192
+// and up to 28% below, where it also cannot join a launch with other segments.
+// V read in place needs a token stride in [1, 2^24) (32-bit offsets within a
+// tile); the copy reads any.
 constexpr int32_t kTransposeRows = 65536;
 inline bool transposes_v(int64_t q_length, int64_t group, int64_t sv_t) {
   return q_length * group >= kTransposeRows || sv_t <= 0 || sv_t >= (1 << 24);

@@ -392,7 +392,13 @@ struct SideJoin {
   int32_t finish() {
     if (!active) return 0;
     active = false;
-    SA_HIP_RETURN(hipEventRecord(p->join, p->side));
+    const hipError_t err = hipEventRecord(p->join, p->side);
+    if (err != hipSuccess) {
+      // Without the event neither the compute stream nor wait_side would
+      // follow these launches.
+      (void)hipStreamSynchronize(p->side);
+      return sa::hip_status(err, "recording the second stream's end");
+    }
     SA_HIP_RETURN(hipStreamWaitEvent(compute, p->join, 0));
     return 0;
   }
@@ -1115,8 +1121,8 @@ std::vector<int> head_group_unit_sizes(int kv_heads, int group_kv, int num_sets)
 //   compute: wait set_ready; per segment [transpose V, where transposes_v
 //         says so: copied always, 20 segments of 300 tokens x 8 heads took
 //         1,483 us a run instead of 1,320, 64 of 64 2,089 instead of 1,613],
-//         one fused update launch over all its queries and keys that writes the output (over
-//         the unit's Q rows) and the LSE; record set_done;
+//         one fused update launch over all its queries and keys that writes
+//         the output (over the unit's Q rows) and the LSE; record set_done;
 //   D2H : wait set_done; output columns back into the host rows, record
 //         set_free.
 // Every byte of Q, K and V crosses the link once.  The launch for unit u + 1
